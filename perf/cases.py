@@ -102,7 +102,8 @@ def draw(rng):
     dist = rng.choice(["uniform", "full", "clustered", "zipf"])
     erase = rng.choice([0.0, 0.1, 0.3])
     c = {"kind": kind, "key_bytes": kb, "dist": dist}
-    wl = rng.randint(4, 16) + (32 if kb == 8 else 0)
+    # the key space is 2^31 (or, 64-bit keys but the skewed ones, 2^62) wide
+    wl = rng.randint(4, 16) + (32 if kb == 8 and dist != "zipf" else 0)
     if kind == "lookup":
         rows = _size(rng, 1 << 14, 1 << 24)
         c.update(rows=rows, batch=_size(rng, max(1 << 10, rows >> 6), 1 << 20),
