@@ -1263,9 +1263,7 @@ inline u32 grouped_lookup_blocks(u64 n) {
   return static_cast<u32>((c + 7) & ~u64(7));
 }
 
-// Wave per query.  Rows of run r count when they are live and no newer run
-// holds the same key (newer versions and tombstones shadow them).  Sums
-// accumulate in 64 bits and are truncated to the value width.
+// Range sums and counts over every run.
 constexpr int kRangeThreads = 256;
 constexpr int kRangeWaves = kRangeThreads / kWave;
 
@@ -1299,131 +1297,384 @@ __host__ __device__ __forceinline__ u32 range_queries_per_wave(u32 runs) {
   return per >= static_cast<u32>(kWave) ? 1u : static_cast<u32>(kWave) / per;
 }
 
-// One wave per round of qw queries.  The lanes first resolve the lower and
-// upper bounds of the round's queries in every run at once (one lane per
-// query, run and side).  A row counts when it is live and no newer run
-// holds its key.  Then, for the whole round at once:
-//   * the rows of every run newer than a query's oldest run with rows are
-//     staged in LDS (decoded keys, tombstone bits) and set bits of a round
-//     filter;
-//   * a count over an oldest run without tombstones takes that run's row
-//     count, minus one for every key whose newest version lies in a newer
-//     run and that the oldest run also holds (one point search per newer
-//     key), plus the newer keys' own newest versions that are live; only
-//     the newer rows are visited;
-//   * otherwise every row of the query's segments is visited, and a row of
-//     a run other than the newest searches the staged keys of the newer
-//     runs when its filter bit is set;
-// with the work items of all queries of the round flattened over the
-// lanes, so a round costs a few memory round trips however many queries
-// it holds.  The count shortcut replaces the visit of the oldest run's
-// rows (one coalesced load per 64 rows) by a point search per newer row
-// (about three dependent round trips), so a query takes it only when its
-// oldest run holds at least kRangeFastRatio times as many rows in the
-// range as the newer runs.  When the staged keys of a round exceed the
-// stage (kRangeStageBytes per wave), its queries are answered one at a
-// time by the whole wave instead.  Sums accumulate in 64 bits and are
-// truncated to the value width.
-constexpr u32 kRangeStageBytes = 8192;   // staged keys per wave, in bytes
-constexpr u32 kRangeFastRatio = 2;
-constexpr u32 kRangeFilterLog = 13;      // filter bits per wave (log2)
-
-template <class K>
-__device__ __forceinline__ u32 range_filter_bit(K key) {
-  u32 x = static_cast<u32>(key);
-  if constexpr (sizeof(K) == 8) x ^= static_cast<u32>(key >> 32);
-  return (x * 0x9E3779B1u) >> (32 - kRangeFilterLog);
+// Queries per wave round of a launch of n queries: fewer than the lanes
+// allow while that keeps fewer than kRangeSpread waves busy (a few thousand
+// queries of a handful of runs would otherwise fill a fraction of the chip;
+// with twice as many waves, narrow queries take a second turn on it).  In a
+// dictionary of more than kRangeWideRows rows, whose queries may be long, the
+// waves are kRangeWideSpread.
+constexpr u64 kRangeSpread = 2048;
+constexpr u64 kRangeWideSpread = 8192;
+constexpr u64 kRangeWideRows = u64(1) << 17;
+inline u32 range_round(u64 n, u32 runs, u64 rows) {
+  const u64 most = range_queries_per_wave(runs);
+  const u64 even = n / (rows > kRangeWideRows ? kRangeWideSpread : kRangeSpread);
+  return static_cast<u32>(even < 1 ? 1 : (even < most ? even : most));
 }
+
+// A query of more work than this (rows that it reads; rows of newer runs,
+// which search the older ones, weigh four) is long: its workgroup's waves
+// share it, in chunks of kRangeNewerStep and kRangeOldStep rows.
+constexpr u32 kRangeLongWork = 1024;
+constexpr u32 kRangeNewerStep = 256;
+constexpr u32 kRangeOldStep = 1024;
+
+// Workgroups that share the long queries of one group of queries: `size` of
+// them, this one being number `rank`.  Where size > 1, acc and left (one each
+// per query of the launch, zero before and after it) gather their sums.
+struct RangeTeam {
+  u32 size, rank;
+  unsigned long long *acc;
+  u32 *left;
+};
+
+// A pointer that was kept in LDS: it points to global memory, which the
+// compiler cannot see by itself (it would use flat accesses, which wait for
+// the LDS accesses in flight too).
+template <class E>
+__device__ __forceinline__ const E *as_global(const E *p) {
+  return (const E *)(const __attribute__((address_space(1))) E *)
+      reinterpret_cast<u64>(p);
+}
+
+// The runs' headers and pointers in LDS (a lane indexes them by its own run).
+template <class T>
+struct RangeRuns {
+  RunMeta meta[kMaxRuns];
+  const typename T::Row *rows_[kMaxRuns];
+  const u32 *dir_[kMaxRuns];
+  __device__ __forceinline__ const typename T::Row *rows(u32 r) const {
+    return as_global(rows_[r]);
+  }
+  __device__ __forceinline__ const u32 *dir(u32 r) const {
+    return as_global(dir_[r]);
+  }
+  __device__ __forceinline__ void load(const RunSet<T> &runs) {
+    if (threadIdx.x < runs.count) {
+      meta[threadIdx.x] = *runs.run[threadIdx.x].meta;
+      rows_[threadIdx.x] = runs.run[threadIdx.x].rows;
+      dir_[threadIdx.x] = runs.run[threadIdx.x].dir;
+    }
+  }
+};
+
+// What row idx of run r adds to its query: its own value (1 for a count, 0
+// for a tombstone) less the value of the next older version of its key, which
+// it shadows.  A key's versions then add up to its newest one's value, each
+// older one being the next older version of exactly one row, so no row has
+// to look for newer versions and the oldest run's rows, usually the most, are
+// only read.  bnd = the query's bounds ([2r] lower, [2r + 1] upper): the rows
+// searched in run s are the query's own, a few of them without the directory.
+// (Two or four rows of a lane in lock step were measured slower.)
+template <class T>
+__device__ __forceinline__ u64 range_row(const RangeRuns<T> &R, const u32 *bnd,
+                                         u32 r, u32 idx, u32 oldest,
+                                         bool count) {
+  using K = typename T::K;
+  using Row = typename T::Row;
+  const Row w = R.rows(r)[idx];
+  u64 v = (T::kw(w) & T::kTomb) ? u64(0) : count ? u64(1) : u64(T::val(w));
+  if (r >= oldest) return v;
+  const K key = decode_key<T>(T::kw(w), idx, R.meta[r].split);
+  const K target = key & T::kLow;
+  for (u32 s = r + 1; s <= oldest; ++s) {
+    u32 lo = bnd[2 * s], hi = bnd[2 * s + 1];
+    if (lo >= hi) continue;
+    const Row *rows = R.rows(s);
+    if (hi - lo > kFindWindow) {
+      const RunMeta &m = R.meta[s];
+      const u32 bucket = static_cast<u32>(key >> (T::kBits - m.dir_bits));
+      if (bucket < m.lo_bucket || bucket > m.hi_bucket) continue;
+      const u32 *dir = R.dir(s);
+      const u32 dlo = dir[bucket], dhi = dir[bucket + 1];
+      lo = dlo > lo ? dlo : lo;
+      hi = dhi < hi ? dhi : hi;
+      // wide buckets (skewed keys): bisect; a bucket's keys share the top bit
+      while (hi > lo + kFindWindow) {
+        const u32 mid = (lo + hi) >> 1;
+        const K km = T::kw(rows[mid]) & T::kLow;
+        if (km == target) {  // one row is left
+          lo = mid;
+          hi = mid + 1;
+        } else if (km < target) {
+          lo = mid + 1;
+        } else {
+          hi = mid;
+        }
+      }
+    }
+    // the window; 8-byte rows in aligned pairs (row arrays carry a spare row,
+    // so the pair of a window's last row is inside the allocation)
+    constexpr u32 kPair = sizeof(Row) == 8 ? 2 : 1;
+    constexpr u32 kSlots = kPair == 2 ? kFindWindow + 2 : kFindWindow;
+    Row x[kSlots];
+    const u32 at0 = kPair == 2 ? (lo & ~1u) : lo;
+#pragma unroll
+    for (u32 i = 0; i < kSlots; i += kPair) {
+      if (at0 + i < hi) {
+        if constexpr (kPair == 2) {
+          const uint4 p = *reinterpret_cast<const uint4 *>(rows + at0 + i);
+          x[i] = T::make(p.x, p.y);
+          x[i + 1] = T::make(p.z, p.w);
+        } else {
+          x[i] = rows[at0 + i];
+        }
+      }
+    }
+    const u32 split = R.meta[s].split;
+    bool found = false;
+#pragma unroll
+    for (u32 i = 0; i < kSlots; ++i) {
+      const u32 at = at0 + i;
+      if (at >= lo && at < hi && decode_key<T>(T::kw(x[i]), at, split) == key) {
+        if (!(T::kw(x[i]) & T::kTomb)) v -= count ? u64(1) : u64(T::val(x[i]));
+        found = true;
+      }
+    }
+    if (found) break;
+  }
+  return v;
+}
+
+// What rows [at, at + n) of run r add to a query together (see range_row), by
+// one wave whose lanes agree on everything but their rows: run by older run,
+// kGroup rows per lane at a time (their directory entries in flight together),
+// the runs' pointers and headers in scalar registers.  A key that lies in the
+// query's range needs no check against its bounds in a run: the directory's
+// rows of its bucket hold it or nothing does.
+template <class T>
+__device__ __forceinline__ u64 range_run_rows(const RangeRuns<T> &R,
+                                              const u32 *bnd, u32 r, u32 at,
+                                              u32 n, u32 oldest, bool count) {
+  using K = typename T::K;
+  using Row = typename T::Row;
+  constexpr int kGroup = sizeof(K) == 4 ? 4 : 2;
+  const u32 lane = lane_id();
+  // (the builtin returns an int: widened as such, a low word with its top
+  // bit set would fill the high word)
+  auto uniform = [](u32 x) -> u32 { return __builtin_amdgcn_readfirstlane(x); };
+  auto uniform_ptr = [&](const auto *p) {
+    const u64 a = reinterpret_cast<u64>(p);
+    const u64 b = u64(uniform(static_cast<u32>(a >> 32))) << 32 |
+                  uniform(static_cast<u32>(a));
+    return as_global(reinterpret_cast<decltype(p)>(b));
+  };
+  const Row *own = uniform_ptr(R.rows(r));
+  const u32 own_split = uniform(R.meta[r].split);
+  u64 acc = 0;
+  for (u32 i0 = 0; i0 < n; i0 += kGroup * kWave) {
+    Row w[kGroup];
+    K key[kGroup];
+    bool open[kGroup];
+#pragma unroll
+    for (int j = 0; j < kGroup; ++j) {
+      const u32 i = i0 + j * kWave + lane;
+      open[j] = i < n;
+      if (open[j]) w[j] = own[at + i];
+    }
+#pragma unroll
+    for (int j = 0; j < kGroup; ++j) {
+      key[j] = 0;
+      if (open[j]) {
+        key[j] = decode_key<T>(T::kw(w[j]), at + i0 + j * kWave + lane,
+                               own_split);
+        if (!(T::kw(w[j]) & T::kTomb)) acc += count ? u64(1) : u64(T::val(w[j]));
+      }
+    }
+    for (u32 s = r + 1; s <= oldest; ++s) {
+      if (uniform(bnd[2 * s]) >= uniform(bnd[2 * s + 1])) continue;
+      const Row *rows = uniform_ptr(R.rows(s));
+      const u32 *dir = uniform_ptr(R.dir(s));
+      const u32 shift = T::kBits - uniform(R.meta[s].dir_bits);
+      const u32 lo_b = uniform(R.meta[s].lo_bucket);
+      const u32 hi_b = uniform(R.meta[s].hi_bucket);
+      u32 lo[kGroup], hi[kGroup];
+#pragma unroll
+      for (int j = 0; j < kGroup; ++j) {
+        const u32 bucket = static_cast<u32>(key[j] >> shift);
+        lo[j] = hi[j] = 0;
+        if (open[j] && bucket >= lo_b && bucket <= hi_b) {
+          lo[j] = dir[bucket];
+          hi[j] = dir[bucket + 1];
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < kGroup; ++j) {
+        const K target = key[j] & T::kLow;
+        u32 a = lo[j], z = hi[j];
+        while (z - a > kFindWindow) {  // wide buckets (skewed keys)
+          const u32 mid = (a + z) >> 1;
+          const K km = T::kw(rows[mid]) & T::kLow;
+          if (km == target) {  // one row is left
+            a = mid;
+            z = mid + 1;
+          } else if (km < target) {
+            a = mid + 1;
+          } else {
+            z = mid;
+          }
+        }
+        Row x[kFindWindow];
+#pragma unroll
+        for (u32 k = 0; k < kFindWindow; ++k)
+          if (a + k < z) x[k] = rows[a + k];
+#pragma unroll
+        for (u32 k = 0; k < kFindWindow; ++k) {
+          if (a + k < z && (T::kw(x[k]) & T::kLow) == target) {
+            if (!(T::kw(x[k]) & T::kTomb))
+              acc -= count ? u64(1) : u64(T::val(x[k]));
+            open[j] = false;
+          }
+        }
+      }
+    }
+  }
+  return acc;
+}
+
+// What chunk c of a long query adds to it: rows of the newer runs (run after
+// run, kRangeNewerStep at a time), then of the oldest, by one wave.
+template <class T>
+__device__ __forceinline__ u64 range_chunk(const RangeRuns<T> &R,
+                                           const u32 *bnd, u32 first,
+                                           u32 oldest, bool count, u64 c,
+                                           u64 newer_chunks) {
+  u64 acc = 0;
+  if (c < newer_chunks) {
+    u64 off = c * kRangeNewerStep;
+    u32 rest = kRangeNewerStep;
+    for (u32 r = first; r < oldest && rest; ++r) {
+      const u32 cnt = bnd[2 * r + 1] - bnd[2 * r];
+      if (off >= cnt) {
+        off -= cnt;
+        continue;
+      }
+      const u32 take = cnt - off < rest ? static_cast<u32>(cnt - off) : rest;
+      acc += range_run_rows<T>(R, bnd, r, bnd[2 * r] + static_cast<u32>(off),
+                               take, oldest, count);
+      rest -= take;
+      off = 0;
+    }
+    return acc;
+  }
+  const u64 a = bnd[2 * oldest] + (c - newer_chunks) * kRangeOldStep;
+  const u64 z = a + kRangeOldStep < bnd[2 * oldest + 1]
+                    ? a + kRangeOldStep
+                    : bnd[2 * oldest + 1];
+  const typename T::Row *rows = R.rows(oldest);
+  auto add = [&](const typename T::Row &w) {
+    if (!(T::kw(w) & T::kTomb)) acc += count ? u64(1) : u64(T::val(w));
+  };
+  u64 i = a + lane_id();
+  for (; i + 3 * kWave < z; i += 4 * kWave) {  // four rows of a lane in flight
+    typename T::Row w[4];
+#pragma unroll
+    for (u32 j = 0; j < 4; ++j) w[j] = rows[i + j * kWave];
+#pragma unroll
+    for (u32 j = 0; j < 4; ++j) add(w[j]);
+  }
+  for (; i < z; i += kWave) add(rows[i]);
+  return acc;
+}
+
 // The range kernel's work on queries [q_begin, q_end) by the calling
-// workgroup, whose waves are wave_id .. of a grid of wave_stride waves
-// (the range kernel's grid, or the serving engine's step kernel taking
-// chunks of queries).  `io` is already staged; every thread of the
-// workgroup calls it.
+// workgroup, number group of a grid of groups (the range kernel's, or the
+// serving engine's step kernel taking chunks of queries), qw queries per wave
+// and round.  `io` is already staged; every thread of the workgroup calls it.
+//
+// The lanes first resolve the bounds of a wave's queries in every run at
+// once (one lane per query, run and side).  The rows of all short queries are
+// then flattened over the lanes (range_row), so a round costs a few memory
+// round trips however many queries it holds; a lane keeps its sum in a
+// register until its next row belongs to another query.  Long queries wait
+// in a list until the workgroup's waves have their short ones, and are then
+// shared by all of them (and by the workgroup's team).  A count takes the rows
+// of a query's oldest run from its bounds when that run has no tombstones.
+// Sums are modulo 2^64 and are truncated to the value width.
+//
+// Bound by the searches, one per newer row and older run (directory entries,
+// then rows), whose lines come from beyond the L2 in a dictionary of tens of
+// megabytes, and by the rows read once.  12,000 sums (or counts) of 2^4 to
+// 2^24 keys' width over 6 million rows in 4 runs, a tenth tombstones: 0.54 ms
+// (9.4 ms when a wave answered each query and every row looked for newer
+// versions, in LDS or, beyond 2048 of them, in global memory); 16,384 counts
+// over one run of 2^20 rows 10 us (15).  A queue of all long queries' chunks
+// for a second launch took 0.38 ms, but its launch made every small call on a
+// large dictionary 3 to 5 us longer.
 template <class T, class IO>
 __device__ __forceinline__ void range_block(const IO &io, u64 q_begin,
                                             u64 q_end, const RunSet<T> &runs,
-                                            u64 wave_id, u64 wave_stride) {
+                                            u64 group, u64 groups, u32 qw,
+                                            const RangeTeam &team) {
   using K = typename T::K;
-  constexpr u32 kRangeCache = kRangeStageBytes / sizeof(K);
   constexpr u32 kSlots =
       2 * kMaxRuns > kWave ? 2 * kMaxRuns : static_cast<u32>(kWave);
+  constexpr u32 kQMax = kWave / 2;  // queries per wave and round
   // s_b[wave][2 * (qi * runs + r) + side]: lower (side 0) and upper (side
   // 1) bound of query qi of the round in run r
   __shared__ u32 s_b[kRangeWaves][kSlots];
-  __shared__ RunMeta s_meta[kMaxRuns];
-  __shared__ K s_cache[kRangeWaves][kRangeCache];
-  __shared__ u32 s_filter[kRangeWaves][(1u << kRangeFilterLog) / 32];
-  __shared__ u32 s_tomb[kRangeWaves][kRangeCache / 32];
-  constexpr u32 kQMax = kWave / 2;  // queries per round (two bounds each)
+  __shared__ RangeRuns<T> R;
   __shared__ typename IO::Slot s_slot[kRangeWaves][kQMax];
   // per query of the round: flags (exists, a <= z, count), plan (first |
-  // oldest << 8 | fast << 16), work and staged-key offsets, accumulator
+  // oldest << 8), work offset and sum
   __shared__ u32 s_flags[kRangeWaves][kQMax];
   __shared__ u32 s_plan[kRangeWaves][kQMax];
   __shared__ u32 s_woff[kRangeWaves][kQMax];
-  __shared__ u32 s_coff[kRangeWaves][kQMax];
-  __shared__ u32 s_stg[kRangeWaves][kQMax];  // newer rows (staged)
-  __shared__ u32 s_wrk[kRangeWaves][kQMax];  // work items
   __shared__ unsigned long long s_acc[kRangeWaves][kQMax];
+  // the round's long queries (wave << 8 | query); round k counts in slot
+  // k % 3 and clears the next one, which no wave can still be reading
+  __shared__ u32 s_list[kRangeWaves * kQMax];
+  __shared__ u32 s_long[3];
   const u32 nr = runs.count;
-  __syncthreads();  // a previous call's readers of s_meta are done
-  if (threadIdx.x < nr) s_meta[threadIdx.x] = *runs.run[threadIdx.x].meta;
+  __syncthreads();  // a previous call's readers of R are done
+  R.load(runs);
+  if (threadIdx.x < 3) s_long[threadIdx.x] = 0;
   __syncthreads();
-  if (nr == 0) {  // no runs: every range is empty
-    const u64 stride = wave_stride * kWave;
-    for (u64 q = q_begin + (wave_id - wave_id % kRangeWaves) * kWave +
-                 threadIdx.x;
-         q < q_end; q += stride) {
-      typename IO::Slot slot;
-      K a, z;
-      bool count_only;
-      io.load(q, slot, a, z, count_only);
-      io.put(slot, typename T::V(0));
-    }
-    return;
-  }
   const u32 lane = lane_id();
   const u32 wave = threadIdx.x / kWave;
-  const u32 per = 2 * nr;  // >= 2: the bounds pass writes every query's
-                           // flags and slot
-  const u32 qw = range_queries_per_wave(nr);
-  const u64 n = q_end;
-  for (u64 q0 = q_begin + wave_id * qw; q0 < n; q0 += wave_stride * qw) {
-    // every bound of the round at once, one lane each
-    for (u32 t = lane; t < qw * per; t += kWave) {
-      const u64 q = q0 + t / per;
-      const u32 r = (t % per) >> 1;
+  const u32 per = 2 * nr;
+  u32 turn = 0;
+  for (u64 g0 = q_begin + group * (kRangeWaves * qw); g0 < q_end;
+       g0 += groups * (kRangeWaves * qw), turn = turn == 2 ? 0 : turn + 1) {
+    const u64 q0 = g0 + u64(wave) * qw;
+    // every bound of the round at once, one lane each (and one per query
+    // when there are no runs: every range is empty)
+    const u32 step = per ? per : 1;
+    for (u32 t = lane; t < qw * step; t += kWave) {
+      const u64 q = q0 + t / step;
+      const u32 r = (t % step) >> 1;
       u32 b = 0;
       u32 flags = 0;
       typename IO::Slot slot{};
-      if (q < n) {
+      if (q < q_end) {
         K a, z;
         bool count_only;
         io.load(q, slot, a, z, count_only);
         flags = 1u | (a <= z ? 2u : 0u) | (count_only ? 4u : 0u);
-        if (a <= z) {
-          const RunView<T> &rv = runs.run[r];
-          const RunMeta m = s_meta[r];
+        if (a <= z && per) {
+          const RunView<T> rv{R.rows(r), R.dir(r), nullptr};
+          const RunMeta m = R.meta[r];
           b = (t & 1) ? run_upper_bound(rv, m, z) : run_lower_bound(rv, m, a);
         }
       }
-      s_b[wave][t] = b;
-      if (t % per == 0) {
-        s_slot[wave][t / per] = slot;
-        s_flags[wave][t / per] = flags;
+      if (per) s_b[wave][t] = b;
+      if (t % step == 0) {
+        s_slot[wave][t / step] = slot;
+        s_flags[wave][t / step] = flags;
       }
     }
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
 
     // ---- plan of query q0 + lane (lanes below qw)
-    u32 work = 0, staged = 0;
+    u32 work = 0;
+    bool is_long = false;
     if (lane < qw) {
       const u32 flags = s_flags[wave][lane];
+      const u32 *bnd = &s_b[wave][lane * per];
       u32 plan = 0;
       u64 base = 0;
       if ((flags & 3u) == 3u) {
-        const u32 *bnd = &s_b[wave][lane * per];
         u32 first = nr, oldest = 0;
         for (u32 r = 0; r < nr; ++r) {
           if (bnd[2 * r] < bnd[2 * r + 1]) {
@@ -1432,287 +1683,137 @@ __device__ __forceinline__ void range_block(const IO &io, u64 q_begin,
           }
         }
         if (first < nr) {
-          u32 newer = 0;
-          for (u32 r = first; r < oldest; ++r) newer += bnd[2 * r + 1] - bnd[2 * r];
-          const u32 old_rows = bnd[2 * oldest + 1] - bnd[2 * oldest];
-          const bool fast = (flags & 4u) && s_meta[oldest].tombs == 0 &&
-                            old_rows >= kRangeFastRatio * newer;
-          staged = newer;
-          work = fast ? newer : newer + old_rows;
-          if (fast) base = old_rows;
-          plan = first | (oldest << 8) | (fast ? 1u << 16 : 0u);
+          u64 newer = 0;
+          for (u32 r = first; r < oldest; ++r)
+            newer += bnd[2 * r + 1] - bnd[2 * r];
+          u32 old_rows = bnd[2 * oldest + 1] - bnd[2 * oldest];
+          plan = first | (oldest << 8);
+          if ((flags & 4u) && R.meta[oldest].tombs == 0) {
+            base = team.rank == 0 ? old_rows : 0;
+            old_rows = 0;
+          }
+          is_long = 4 * newer + old_rows > kRangeLongWork;
+          if (is_long)
+            s_list[atomicAdd(&s_long[turn], 1u)] = wave << 8 | lane;
+          else if (team.rank == 0)
+            work = static_cast<u32>(newer + old_rows);
         }
       }
       s_plan[wave][lane] = plan;
       s_acc[wave][lane] = base;
     }
     const u32 work_inc = wave_inclusive_scan(work);
-    const u32 staged_inc = wave_inclusive_scan(staged);
-    if (lane < qw) {
-      s_woff[wave][lane] = work_inc - work;
-      s_coff[wave][lane] = staged_inc - staged;
-      s_stg[wave][lane] = staged;
-      s_wrk[wave][lane] = work;
-    }
+    if (lane < qw) s_woff[wave][lane] = work_inc - work;
+    const u32 wend = __shfl(work_inc, kWave - 1, kWave);
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
 
-    // one query by the whole wave: every row of its segments, the newer
-    // runs searched in place (its newer rows exceed the stage)
-    auto alone = [&](u32 qi) {
-      const u64 q = q0 + qi;
-      if (q >= n) return;
-      typename IO::Slot slot;
-      K a, z;
-      bool count_only;
-      io.load(q, slot, a, z, count_only);
-      if (a > z) {
-        if (lane == 0) io.put(slot, typename T::V(0));
-        return;
-      }
-      const u32 *bnd = &s_b[wave][qi * per];  // [2r] lower, [2r + 1] upper
-      // the newest run with rows in the range
-      u32 first = nr;
-      for (u32 r = 0; r < nr; ++r) {
-        if (bnd[2 * r] < bnd[2 * r + 1]) {
-          first = r;
-          break;
-        }
-      }
+    // rows of the short queries, flattened query after query, run after run
+    if (wend) {
+      u32 qi = 0;
       u64 acc = 0;
-      u32 skip = nr;  // a run counted without a scan
-      if (first < nr && count_only && s_meta[first].tombs == 0) {
-        if (lane == 0) acc = bnd[2 * first + 1] - bnd[2 * first];
-        skip = first;
-      }
-      u32 total = 0, oldest = first;
-      for (u32 r = first; r < nr; ++r) {
-        const u32 cnt = bnd[2 * r + 1] - bnd[2 * r];
-        if (r != skip) total += cnt;
-        if (cnt) oldest = r;
-      }
-      // stage the keys of runs first .. oldest - 1, run after run
-      u32 cached = 0;
-      for (u32 r = first; r < oldest; ++r) cached += bnd[2 * r + 1] - bnd[2 * r];
-      const bool use_cache = cached <= kRangeCache;
-      u32 *filter = s_filter[wave];
-      if (cached) {
-        // (the previous query's reads of s_cache and s_filter are done)
-        __builtin_amdgcn_wave_barrier();
-        for (u32 i = lane; i < (1u << kRangeFilterLog) / 32; i += kWave)
-          filter[i] = 0;
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        for (u32 f = lane; f < cached; f += kWave) {
-          u32 r = first, off = f;
-          while (off >= bnd[2 * r + 1] - bnd[2 * r]) {
-            off -= bnd[2 * r + 1] - bnd[2 * r];
-            ++r;
-          }
-          const u32 idx = bnd[2 * r] + off;
-          const K key = decode_key<T>(T::kw(runs.run[r].rows[idx]), idx,
-                                      s_meta[r].split);
-          if (use_cache) s_cache[wave][f] = key;
-          const u32 bit = range_filter_bit(key);
-          atomicOr(&filter[bit >> 5], 1u << (bit & 31));
+      if (lane < wend) {
+        u32 hi = qw;
+        while (hi - qi > 1) {  // the last query whose offset is <= lane
+          const u32 mid = (qi + hi) >> 1;
+          if (s_woff[wave][mid] <= lane) qi = mid;
+          else hi = mid;
         }
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
       }
-      for (u32 f = lane; f < total; f += kWave) {
-        // run r and row idx of flattened row f
-        u32 r = first, off = f;
-        while (true) {
-          if (r != skip) {
-            const u32 cnt = bnd[2 * r + 1] - bnd[2 * r];
-            if (off < cnt) break;
-            off -= cnt;
-          }
-          ++r;
+      for (u32 f = lane; f < wend; f += kWave) {
+        u32 next = qi;
+        while (next + 1 < qw && s_woff[wave][next + 1] <= f) ++next;
+        if (next != qi) {
+          if (acc)
+            atomicAdd(&s_acc[wave][qi], static_cast<unsigned long long>(acc));
+          acc = 0;
+          qi = next;
         }
-        const u32 idx = bnd[2 * r] + off;
-        const RunView<T> &rv = runs.run[r];
-        const typename T::Row w = rv.rows[idx];
-        if (T::kw(w) & T::kTomb) continue;
-        bool shadowed = false;
-        const K key = decode_key<T>(T::kw(w), idx, s_meta[r].split);
-        const u32 bit = range_filter_bit(key);
-        if (r > first && ((filter[bit >> 5] >> (bit & 31)) & 1u)) {
-          u32 base = 0;  // staged keys of runs first .. s - 1
-          for (u32 s = first; s < r && !shadowed; ++s) {
-            u32 l2 = bnd[2 * s], h2 = bnd[2 * s + 1];
-            const u32 cnt = h2 - l2;
-            if (!cnt) continue;
-            if (use_cache) {
-              const K *c = &s_cache[wave][base];
-              u32 lo = 0, hi = cnt;
-              while (lo < hi) {
-                const u32 mid = (lo + hi) >> 1;
-                if (c[mid] < key) lo = mid + 1;
-                else hi = mid;
-              }
-              shadowed = lo < cnt && c[lo] == key;
-              base += cnt;
-              continue;
-            }
-            const RunView<T> &nv = runs.run[s];
-            const u32 ns = s_meta[s].split;
-            const u32 end = h2;
-            while (l2 < h2) {
-              const u32 mid = (l2 + h2) >> 1;
-              if (decode_key<T>(T::kw(nv.rows[mid]), mid, ns) < key)
-                l2 = mid + 1;
-              else
-                h2 = mid;
-            }
-            if (l2 < end && decode_key<T>(T::kw(nv.rows[l2]), l2, ns) == key)
-              shadowed = true;
-          }
-        }
-        if (!shadowed) acc += count_only ? u64(1) : u64(T::val(w));
-      }
-      acc = wave_sum_u64(acc);
-      if (lane == 0) io.put(slot, static_cast<typename T::V>(acc));
-        };
-
-    // query of a flattened index f among queries [g0, g1): the last query
-    // whose offset is <= f
-    auto query_in = [&](const u32 *off, u32 g0, u32 g1, u32 f) {
-      u32 lo = g0, hi = g1;
-      while (hi - lo > 1) {
-        const u32 mid = (lo + hi) >> 1;
-        if (off[mid] <= f) lo = mid;
-        else hi = mid;
-      }
-      return lo;
-    };
-    u32 *filter = s_filter[wave];
-    for (u32 g0 = 0; g0 < qw;) {
-      // the group [g0, g1): consecutive queries whose newer rows fit the
-      // stage together
-      const u32 cbase = s_coff[wave][g0];
-      u32 g1 = g0;
-      while (g1 < qw &&
-             s_coff[wave][g1] + s_stg[wave][g1] - cbase <= kRangeCache)
-        ++g1;
-      if (g1 == g0) {
-        alone(g0);
-        ++g0;
-        __builtin_amdgcn_wave_barrier();
-        continue;
-      }
-      const u32 wbase = s_woff[wave][g0];
-      const u32 wend = s_woff[wave][g1 - 1] + s_wrk[wave][g1 - 1];
-      const u32 ncache = s_coff[wave][g1 - 1] + s_stg[wave][g1 - 1] - cbase;
-      if (ncache) {
-        // (the previous group's reads of the stage and filter are done)
-        __builtin_amdgcn_wave_barrier();
-        for (u32 i = lane; i < (1u << kRangeFilterLog) / 32; i += kWave)
-          filter[i] = 0;
-        for (u32 i = lane; i < kRangeCache / 32; i += kWave)
-          s_tomb[wave][i] = 0;
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        // stage the newer rows: query after query, run after run
-        for (u32 f = cbase + lane; f < cbase + ncache; f += kWave) {
-          const u32 qi = query_in(s_coff[wave], g0, g1, f);
-          const u32 *bnd = &s_b[wave][qi * per];
-          u32 r = s_plan[wave][qi] & 0xffu, off = f - s_coff[wave][qi];
-          while (off >= bnd[2 * r + 1] - bnd[2 * r]) {
-            off -= bnd[2 * r + 1] - bnd[2 * r];
-            ++r;
-          }
-          const u32 idx = bnd[2 * r] + off;
-          const typename T::K w = T::kw(runs.run[r].rows[idx]);
-          const K key = decode_key<T>(w, idx, s_meta[r].split);
-          const u32 ci = f - cbase;
-          s_cache[wave][ci] = key;
-          if (w & T::kTomb) atomicOr(&s_tomb[wave][ci >> 5], 1u << (ci & 31));
-          const u32 bit = range_filter_bit(key);
-          atomicOr(&filter[bit >> 5], 1u << (bit & 31));
-        }
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-      }
-      // whether a run newer than r (from `first` on) of query qi holds key
-      auto newer_holds = [&](u32 qi, u32 first, u32 r, K key) {
-        const u32 *bnd = &s_b[wave][qi * per];
-        u32 base = s_coff[wave][qi] - cbase;
-        for (u32 s2 = first; s2 < r; ++s2) {
-          const u32 cnt = bnd[2 * s2 + 1] - bnd[2 * s2];
-          if (!cnt) continue;
-          const K *c = &s_cache[wave][base];
-          u32 lo = 0, hi = cnt;
-          while (lo < hi) {
-            const u32 mid = (lo + hi) >> 1;
-            if (c[mid] < key) lo = mid + 1;
-            else hi = mid;
-          }
-          if (lo < cnt && c[lo] == key) return true;
-          base += cnt;
-        }
-        return false;
-      };
-      for (u32 f = wbase + lane; f < wend; f += kWave) {
-        const u32 qi = query_in(s_woff[wave], g0, g1, f);
         const u32 plan = s_plan[wave][qi];
-        const u32 first = plan & 0xffu, oldest = (plan >> 8) & 0xffu;
-        const bool fast = (plan >> 16) & 1u;
-        const bool count = (s_flags[wave][qi] & 4u) != 0;
         const u32 *bnd = &s_b[wave][qi * per];
-        u32 r = first, off = f - s_woff[wave][qi];
+        u32 r = plan & 0xffu, off = f - s_woff[wave][qi];
         while (off >= bnd[2 * r + 1] - bnd[2 * r]) {
           off -= bnd[2 * r + 1] - bnd[2 * r];
           ++r;
         }
-        const u32 idx = bnd[2 * r] + off;
-        u64 contrib = 0;
-        if (fast) {
-          // a newer row: staged at the same position within its query
-          const u32 ci = s_coff[wave][qi] - cbase + (f - s_woff[wave][qi]);
-          const K key = s_cache[wave][ci];
-          if (!newer_holds(qi, first, r, key)) {
-            const bool tomb = (s_tomb[wave][ci >> 5] >> (ci & 31)) & 1u;
-            typename T::Row row;
-            const bool in_oldest =
-                run_find(runs.run[oldest], s_meta[oldest], key, row) !=
-                0xffffffffu;
-            contrib = u64(tomb ? 0 : 1) - u64(in_oldest ? 1 : 0);
-          }
-        } else {
-          const typename T::Row w = runs.run[r].rows[idx];
-          if (!(T::kw(w) & T::kTomb)) {
-            const K key = decode_key<T>(T::kw(w), idx, s_meta[r].split);
-            const u32 bit = range_filter_bit(key);
-            const bool maybe =
-                r > first && ((filter[bit >> 5] >> (bit & 31)) & 1u);
-            if (!(maybe && newer_holds(qi, first, r, key)))
-              contrib = count ? u64(1) : u64(T::val(w));
-          }
-        }
-        if (contrib)
-          atomicAdd(&s_acc[wave][qi], static_cast<unsigned long long>(contrib));
+        acc += range_row<T>(R, bnd, r, bnd[2 * r] + off, plan >> 8,
+                            (s_flags[wave][qi] & 4u) != 0);
       }
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-      if (lane >= g0 && lane < g1 && (s_flags[wave][lane] & 1u))
-        io.put(s_slot[wave][lane],
-               static_cast<typename T::V>(s_acc[wave][lane]));
-      __builtin_amdgcn_wave_barrier();
-      g0 = g1;
+      // one addition per wave when its lanes end in one query
+      const u32 lead = __builtin_amdgcn_readfirstlane(qi);
+      if (ballot(qi != lead && acc) == 0) {
+        acc = wave_sum_u64(acc);
+        if (lane == 0 && acc)
+          atomicAdd(&s_acc[wave][lead], static_cast<unsigned long long>(acc));
+      } else if (acc) {
+        atomicAdd(&s_acc[wave][qi], static_cast<unsigned long long>(acc));
+      }
     }
     __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    if (lane < qw && !is_long && team.rank == 0 && (s_flags[wave][lane] & 1u))
+      io.put(s_slot[wave][lane],
+             static_cast<typename T::V>(s_acc[wave][lane]));
+
+    // ---- the workgroup's long queries, by all its waves
+    if (threadIdx.x == 0) s_long[turn == 2 ? 0 : turn + 1] = 0;
+    __syncthreads();
+    const u32 longs = s_long[turn];
+    if (!longs) continue;
+    for (u32 l = 0; l < longs; ++l) {
+      const u32 id = s_list[l], w = id >> 8, qi = id & 0xffu;
+      const u32 *bnd = &s_b[w][qi * per];
+      const u32 first = s_plan[w][qi] & 0xffu, oldest = s_plan[w][qi] >> 8;
+      const bool count = (s_flags[w][qi] & 4u) != 0;
+      u64 newer = 0;
+      for (u32 r = first; r < oldest; ++r) newer += bnd[2 * r + 1] - bnd[2 * r];
+      const u64 old_rows = count && R.meta[oldest].tombs == 0
+                               ? 0
+                               : bnd[2 * oldest + 1] - bnd[2 * oldest];
+      const u64 nc = (newer + kRangeNewerStep - 1) / kRangeNewerStep;
+      const u64 chunks = nc + (old_rows + kRangeOldStep - 1) / kRangeOldStep;
+      u64 acc = 0;
+      for (u64 c = u64(team.rank) * kRangeWaves + wave; c < chunks;
+           c += u64(team.size) * kRangeWaves)
+        acc += range_chunk<T>(R, bnd, first, oldest, count, c, nc);
+      acc = wave_sum_u64(acc);
+      if (lane == 0 && acc)
+        atomicAdd(&s_acc[w][qi], static_cast<unsigned long long>(acc));
+    }
+    __syncthreads();
+    if (threadIdx.x < longs) {
+      const u32 id = s_list[threadIdx.x], w = id >> 8, qi = id & 0xffu;
+      u64 sum = s_acc[w][qi];
+      bool last = true;
+      if (team.size > 1) {
+        // The sum must have taken this workgroup's share before `left`
+        // counts it.  The value that the addition returns is waited for
+        // instead of a fence, which would write back and empty the L2.
+        const u64 q = g0 + u64(w) * qw + qi;
+        u64 before =
+            atomicAdd(&team.acc[q], static_cast<unsigned long long>(sum));
+        asm volatile("" : "+v"(before) : : "memory");
+        last = atomicAdd(&team.left[q], 1u) == team.size - 1;
+        if (last) {
+          sum = atomicExch(&team.acc[q], 0ull);
+          atomicExch(&team.left[q], 0u);
+        }
+      }
+      if (last) io.put(s_slot[w][qi], static_cast<typename T::V>(sum));
+    }
+    __syncthreads();  // the next round writes the bounds and the list again
   }
 }
 
+// Teams of team.size consecutive workgroups (team.rank is set here).
 template <class T, class IO>
-__global__ __launch_bounds__(kRangeThreads) void range_kernel(IO io_arg, u64 n,
-                                                              RunSet<T> runs) {
+__global__ __launch_bounds__(kRangeThreads) void range_kernel(
+    IO io_arg, u64 n, RunSet<T> runs, u32 qw, RangeTeam team) {
   __shared__ __align__(16) char s_io[IO::kStageBytes ? IO::kStageBytes : 16];
   const IO io = io_arg.stage(s_io);  // range_block's first barrier orders it
-  range_block<T, IO>(io, 0, n, runs,
-                     u64(blockIdx.x) * kRangeWaves + threadIdx.x / kWave,
-                     u64(gridDim.x) * kRangeWaves);
+  team.rank = blockIdx.x % team.size;
+  range_block<T, IO>(io, 0, n, runs, blockIdx.x / team.size,
+                     gridDim.x / team.size, qw, team);
 }
 
 // Smallest live key >= query, all-ones when there is none.

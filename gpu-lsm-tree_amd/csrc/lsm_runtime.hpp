@@ -333,19 +333,39 @@ class LsmT : public HandleBase {
     order_.begin(s);
     if (range_compaction_pays(n)) compact_runs(s);
     const RunSet<T> set = run_set();
-    const u64 waves = (n + range_queries_per_wave(set.count) - 1) /
-                      range_queries_per_wave(set.count);
     ProfRec rec{};
     if (profiling_) rec = prof_begin(3, s, n);
-    range_kernel<T><<<grid_for(waves, kRangeWaves, 1u << 16), kRangeThreads, 0,
-                      s>>>(PlainRange<T>{lo, hi, out, count_only ? 1 : 0}, n,
-                           set);
-    GD_LAUNCH_CHECK();
+    launch_ranges(PlainRange<T>{lo, hi, out, count_only ? 1 : 0}, n, set, s);
     if (profiling_) {
       rec.runs = set.count;
       prof_end(rec, s);
     }
     order_.end(s);
+  }
+
+  // Answers n ranges over the runs of `set` on stream s.  A few queries of a
+  // large dictionary, any of which may be most of it, get a team of
+  // workgroups each: up to kRangeTeamBlocks in all, for at most
+  // kRangeTeamQueries queries and more than kRangeWideRows rows (fewer rows
+  // take one workgroup some tens of microseconds).  The teams' sums are the
+  // handle's own buffer, zero between calls (a handle's calls are ordered); a
+  // stream under capture gets none, as a graph would go on using it after
+  // the call.
+  static constexpr u32 kRangeTeamQueries = 2048;
+  static constexpr u32 kRangeTeamBlocks = 512;
+
+  template <class IO>
+  void launch_ranges(const IO &io, u64 n, const RunSet<T> &set,
+                     hipStream_t s) {
+    u64 rows = 0;
+    for (const auto &r : runs_) rows += r.rows_ub;
+    const u32 qw = range_round(n, set.count, rows);
+    const u64 waves = (n + qw - 1) / qw;
+    const u32 groups = grid_for(waves, kRangeWaves, 1u << 16);
+    const RangeTeam team = range_team(n, groups, rows, s);
+    range_kernel<T, IO><<<groups * team.size, kRangeThreads, 0, s>>>(
+        io, n, set, qw, team);
+    GD_LAUNCH_CHECK();
   }
 
   void successor(const K *q, u64 n, K *out, hipStream_t s) {
@@ -842,7 +862,8 @@ class LsmT : public HandleBase {
 
   u32 carry_status() const { return status_; }
   u64 resident_bytes() const {
-    return pool_.held_bytes() + merge_pool_.held_bytes();
+    return pool_.held_bytes() + merge_pool_.held_bytes() +
+           range_pool_.held_bytes();
   }
   void memory(gd_memory_stats *out) const {
     out->held_bytes = resident_bytes();
@@ -990,6 +1011,37 @@ class LsmT : public HandleBase {
     pending_batches_ = 0;
     failed_ = false;
     status_ = 0;
+  }
+
+  // The team of each of the `groups` workgroups of n ranges on stream s.
+  RangeTeam range_team(u64 n, u32 groups, u64 rows, hipStream_t s) {
+    RangeTeam team{1, 0, nullptr, nullptr};
+    if (n > kRangeTeamQueries || rows <= kRangeWideRows ||
+        2 * groups > kRangeTeamBlocks)
+      return team;
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &capturing) != hipSuccess) {
+      (void)hipGetLastError();
+      return team;
+    }
+    if (capturing != hipStreamCaptureStatusNone) return team;
+    if (!range_sums_) {
+      const u64 bytes =
+          kRangeTeamQueries * (sizeof(unsigned long long) + sizeof(u32));
+      u32 *sums = nullptr;
+      try {
+        sums = static_cast<u32 *>(range_pool_.get(bytes));
+      } catch (const Error &) {
+        return team;  // no memory for it: a workgroup per group
+      }
+      zero_two_kernel<<<8, 256, 0, s>>>(sums, bytes / sizeof(u32), nullptr, 0);
+      GD_LAUNCH_CHECK();
+      range_sums_ = sums;
+    }
+    team.size = kRangeTeamBlocks / groups;
+    team.acc = reinterpret_cast<unsigned long long *>(range_sums_);
+    team.left = range_sums_ + 2 * kRangeTeamQueries;
+    return team;
   }
 
   // The pool for work on stream s (merges in serving mode have their own).
@@ -1410,6 +1462,10 @@ class LsmT : public HandleBase {
   PoolUsage usage_;
   DevicePool pool_{&usage_};
   DevicePool merge_pool_{&usage_};
+  // the sums of range teams (their own pool: they are used on the stream of
+  // the queries, which may be another than the pool's)
+  DevicePool range_pool_{&usage_};
+  u32 *range_sums_ = nullptr;
   OperationOrder order_;
   std::vector<Run> runs_;  // newest first
   u32 pending_batches_ = 0;

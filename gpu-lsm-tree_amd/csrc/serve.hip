@@ -331,8 +331,9 @@ __global__ __launch_bounds__(lsm::kRangeThreads) void step_query_kernel(
     } else {
       const u64 r0 = u64(item - lc) * kStepRangeChunk;
       lsm::range_block<T, PieceRange<T>>(
-          rio, r0, std::min<u64>(n_rng, r0 + kStepRangeChunk), runs,
-          threadIdx.x / kWave, lsm::kRangeWaves);
+          rio, r0, std::min<u64>(n_rng, r0 + kStepRangeChunk), runs, 0, 1,
+          lsm::range_queries_per_wave(runs.count),
+          lsm::RangeTeam{1, 0, nullptr, nullptr});
     }
   }
 }
@@ -882,12 +883,9 @@ class Server : public ServerBase {
     }
     if (n_rng) {
       // counts and sums share the kernel: each request chooses its own
-      const u64 waves = (n_rng + lsm::range_queries_per_wave(snap.count) - 1) /
-                        lsm::range_queries_per_wave(snap.count);
-      lsm::range_kernel<T><<<grid_for(waves, lsm::kRangeWaves, 1u << 16),
-                             lsm::kRangeThreads, 0, qs_>>>(
-          PieceRange<T>{dev_rng, static_cast<u32>(rng.size())}, n_rng, snap);
-      GD_LAUNCH_CHECK();
+      lsm_.launch_ranges(
+          PieceRange<T>{dev_rng, static_cast<u32>(rng.size())}, n_rng, snap,
+          qs_);
     }
     GD_HIP(hipEventCreateWithFlags(&st.queries_done, hipEventDisableTiming));
     GD_HIP(hipEventRecord(st.queries_done, qs_));
