@@ -25,6 +25,7 @@
 #pragma once
 
 #include "device_utils.hpp"
+#include "radix_sort.hpp"
 
 namespace gdict {
 namespace lsm {
@@ -256,9 +257,10 @@ __global__ __launch_bounds__(kFinThreads) void finalize_batch_kernel(
     const typename T::V *__restrict__ values,
     const u8 *__restrict__ erase_flags, int mode,
     typename T::Row *__restrict__ out, RunMeta *meta, u32 *__restrict__ dir,
-    u32 dir_bits, u64 *status, u32 *ticket) {
+    u32 dir_bits, u64 *status, u32 *ticket, rs::Gate gate) {
   using K = typename T::K;
   using V = typename T::V;
+  if (gate.closed()) return;
   __shared__ u32 s_tile;
   __shared__ u32 s_off[kFinItems][kFinWaves];
   __shared__ u32 s_total;

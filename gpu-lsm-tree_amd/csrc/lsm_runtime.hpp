@@ -3,9 +3,10 @@
 //
 // Replaces class GPULSMOpt (GPULSMOpt.cuh:5599-7805).  The observable
 // contract is the reference's; the structure is this library's own:
-//   * every admitted tile (<= batch_capacity keys) is sorted on the GPU by a
-//     onesweep LDS radix sort (one fused workgroup for <= 4096 keys) and
-//     becomes an immutable sorted run, so reads never scan unsorted rows;
+//   * every admitted tile (<= batch_capacity keys) is sorted on the GPU (a
+//     partition by its top varying byte, then a workgroup per byte value in
+//     LDS; one fused workgroup for <= 4096 keys) and becomes an immutable
+//     sorted run, so reads never scan unsorted rows;
 //   * runs merge pairwise (merge-path partitioned, streamed through LDS)
 //     whenever the older neighbour is no larger than the newer one, which is
 //     a binary counter for equal batches: log2(N/b) merges per row and at
@@ -24,6 +25,7 @@
 #include <string>
 #include <vector>
 
+#include "batch_sort.hpp"
 #include "host_common.hpp"
 #include "kway_merge.hpp"
 #include "lsm_kernels.hpp"
@@ -1097,9 +1099,13 @@ class LsmT : public HandleBase {
       GD_LAUNCH_CHECK();
       return r;
     }
-    if constexpr (sizeof(K) == 4) {
-      if (tuning_.segmented_admission == 1 && n > 16384)
-        return segmented_run(keys, values, flags, n, mode, s, r);
+    if (tuning_.segmented_admission == 1) {
+      if constexpr (sizeof(K) == 4) {
+        if (n > 16384) return segmented_run(keys, values, flags, n, mode, s, r);
+      }
+      // (a larger build's digits would not fit the LDS)
+      if (n <= kMaximumOperationTile)
+        return batch_run(keys, values, flags, n, mode, s, r);
     }
     const u32 fin_tiles = (n + kFinTile - 1) / kFinTile;
     const u64 sort_words = rs::control_words(n, rs::passes_for<K>());
@@ -1117,8 +1123,36 @@ class LsmT : public HandleBase {
     finalize_batch_kernel<T><<<fin_tiles, kFinThreads, 0, s>>>(
         ka.get(), va.get(), n, values, flags, mode, r.rows, r.meta(),
         r.entries(), r.max_bits, reinterpret_cast<u64 *>(fin_ctrl + 64),
-        fin_ctrl);
+        fin_ctrl, rs::Gate{});
     GD_LAUNCH_CHECK();
+    return r;
+  }
+
+  // Sorts a batch into run r through batch_sort.hpp.
+  Run batch_run(const K *keys, const V *values, const u8 *flags, u32 n,
+                int mode, hipStream_t s, Run r) {
+    bs::Scratch<T> x{};
+    Lease<K> ka, kb;
+    Lease<V> vals;
+    Lease<u32> pa, pb, ctrl;
+    if (n > bs::PieceShape<K, V>::kCap) {
+      ka = Lease<K>(pool_, n);
+      kb = Lease<K>(pool_, n);
+      vals = Lease<V>(pool_, n);
+      pa = Lease<u32>(pool_, n);
+      pb = Lease<u32>(pool_, n);
+      ctrl = Lease<u32>(pool_, bs::Layout<K>(n).words);
+      x = {ka.get(), kb.get(), vals.get(), pa.get(), pb.get(), ctrl.get()};
+    }
+    bs::LsmEmit<T> emit{};
+    emit.values = values;
+    emit.flags = flags;
+    emit.mode = mode;
+    emit.out = r.rows;
+    emit.meta = r.meta();
+    emit.dir = r.entries();
+    emit.dir_bits = r.max_bits;
+    GD_HIP(bs::admit_batch<T>(keys, n, x, emit, s, tuning_.sort_block));
     return r;
   }
 
@@ -1418,8 +1452,7 @@ class LsmT : public HandleBase {
 
   u64 batch_capacity_ = 1;
   u64 capacity_ = 0;
-  // segmented admission (1) for 32-bit batches; 64-bit batches always take
-  // the radix passes
+  // segmented admission (1), or the radix passes (2)
   gd_lsm_tuning tuning_{3, 12, 0, 18, static_cast<u32>(T::kSmallTile), 10,
                         1, 512, kMaxWay, 2};
 

@@ -26,6 +26,17 @@ constexpr int passes_for() {
   return static_cast<int>(sizeof(K));
 }
 
+// Whether a launch runs at all, decided on the device: a launch with a gate
+// runs only if (*value > limit) == above (an earlier launch left *value).
+struct Gate {
+  const u32 *value;  // null: always
+  u32 limit;
+  bool above;
+  __device__ __forceinline__ bool closed() const {
+    return value && (*value > limit) != above;
+  }
+};
+
 // Digit histograms.  A block counts 16 keys per thread per round in LDS
 // (the 16 loads are issued together), then adds its counts into one of
 // kHistRows partial rows (row = block % kHistRows), so at most
@@ -45,7 +56,9 @@ inline u32 hist_blocks_for(u64 n) {
 // first .. first + kPasses - 1, digit p = (key >> 8p) & 0xff.
 template <class K, int kPasses>
 static __global__ __launch_bounds__(kThreads) void histogram_kernel(
-    const K *__restrict__ keys, u32 n, u32 first, u32 *__restrict__ rows) {
+    const K *__restrict__ keys, u32 n, u32 first, u32 *__restrict__ rows,
+    Gate gate) {
+  if (gate.closed()) return;
   __shared__ u32 s_hist[kPasses][kRadix];
   for (int i = threadIdx.x; i < kPasses * kRadix; i += kThreads)
     (&s_hist[0][0])[i] = 0;
@@ -79,9 +92,12 @@ static __global__ __launch_bounds__(kThreads) void histogram_kernel(
 }
 
 // Sums the kHistRows partial rows of pass blockIdx.x and writes the
-// exclusive scan over digits -> global digit offsets.
+// exclusive scan over digits -> global digit offsets.  constant[p] (nullable,
+// zero before) = 1 when all n keys share the pass's digit.
 static __global__ __launch_bounds__(kRadix) void scan_kernel(
-    const u32 *__restrict__ rows, u32 passes, u32 *__restrict__ offsets) {
+    const u32 *__restrict__ rows, u32 passes, u32 *__restrict__ offsets,
+    Gate gate = Gate{}, u32 *constant = nullptr, u32 n = 0) {
+  if (gate.closed()) return;
   __shared__ u32 scratch[kRadix / kWave + 1];
   const u32 p = blockIdx.x;
   u32 c[kHistRows];
@@ -92,6 +108,7 @@ static __global__ __launch_bounds__(kRadix) void scan_kernel(
 #pragma unroll
   for (int r = 0; r < kHistRows; ++r) v += c[r];
   offsets[p * kRadix + threadIdx.x] = block_exclusive_scan<kRadix>(v, scratch);
+  if (constant && v == n) constant[p] = 1;
 }
 
 // Payload policies of a digit pass: payload(idx, valid, key, shift)
@@ -112,20 +129,55 @@ struct PayloadPos {  // the input position
   }
 };
 
-// One digit pass.  status has tiles*kRadix words and must be zero;
-// *ticket must be zero.  kBlock threads (256 or 512) x kItems keys per
-// tile; threads below 256 own one digit each for the per-digit bookkeeping.
-template <class K, class Payload, int kItems, int kBlock>
+// Keys and payloads of a pass: src.load(idx, valid, shift, key, val).
+template <class K, class Payload>
+struct ArraySource {
+  const K *keys;
+  Payload payload;
+  __device__ __forceinline__ void load(u64 idx, bool valid, u32 shift, K &key,
+                                       u32 &val) const {
+    key = valid ? keys[idx] : ~K(0);
+    val = payload(idx, valid, key, shift);
+  }
+};
+
+// One digit pass: the digit and where its keys go.
+struct PassPlan {
+  u32 shift;               // the digit's shift, or (not null)
+  const u32 *shift_dev;    // where an earlier launch left it
+  // Passes compiled with a gate (kGated) may not run: when it is closed, or
+  // when pair (not null) says that this pass's and its partner's digits are
+  // constant, so that the two would move nothing (passes 2q and 2q + 1 leave
+  // the batch in the buffer that it came in).
+  Gate gate;
+  const u32 *pair;
+  // the digits' starts, or their totals (scanned here)
+  const u32 *digit_offsets, *digit_totals;
+  // per-tile digit prefixes of the input (tile_prefix[d * tiles + t]: keys of
+  // digit d in tiles before t): the tiles are then independent.  Without
+  // them they chain their offsets: status (tiles * kRadix words) and *ticket
+  // start at zero.
+  const u32 *tile_prefix;
+  u64 *status;
+  u32 *ticket;
+  u32 *dest;               // nullable: each input element's place
+};
+
+// kBlock threads x kItems keys per tile; threads below 256 own one digit each
+// for the per-digit bookkeeping.
+template <class K, class V, class Source, int kItems, int kBlock, bool kGated>
 __global__ __launch_bounds__(kBlock) void onesweep_kernel(
-    const K *__restrict__ keys_in, Payload payload,
-    K *__restrict__ keys_out, u32 *__restrict__ vals_out, u32 n,
-    u32 shift_arg, const u32 *__restrict__ digit_offsets, u64 *status,
-    u32 *ticket, u32 *__restrict__ dest_out, const u32 *shift_dev,
-    const u32 *__restrict__ tile_prefix) {
+    Source src, K *__restrict__ keys_out, V *__restrict__ vals_out, u32 n,
+    PassPlan plan) {
   constexpr int kTile = kBlock * kItems;
-  // the digit shift: an argument, or computed on the device by an earlier
-  // launch
-  const u32 shift = shift_dev ? *shift_dev : shift_arg;
+  // (an ungated pass does not spend the loads on it: 2 us of 37 at 3 million
+  // 64-bit keys)
+  if constexpr (kGated) {
+    if (plan.gate.closed()) return;
+    if (plan.pair && plan.pair[0] && plan.pair[1]) return;
+  }
+  const u32 *tile_prefix = plan.tile_prefix;
+  const u32 shift = plan.shift_dev ? *plan.shift_dev : plan.shift;
   constexpr int kBlockWaves = kBlock / kWave;
   __shared__ u32 s_tile;
   __shared__ u32 s_wave_hist[kBlockWaves][kRadix];
@@ -133,30 +185,33 @@ __global__ __launch_bounds__(kBlock) void onesweep_kernel(
   __shared__ u32 s_global_base[kRadix];
   __shared__ u32 s_scan[kBlockWaves + 1];
   __shared__ K s_keys[kTile];
-  __shared__ u32 s_vals[kTile];
+  __shared__ V s_vals[kTile];
 
   const u32 tid = threadIdx.x;
   const u32 lane = lane_id();
   const u32 wave = tid / kWave;
-  // with precomputed per-tile digit prefixes (tile_prefix[d * tiles + t]:
-  // keys of digit d in tiles before t; digit_offsets then holds the digit
-  // totals) the tiles are independent: no ticket and no look-back
-  if (tid == 0) s_tile = tile_prefix ? blockIdx.x : atomicAdd(ticket, 1u);
+  if (tid == 0) s_tile = tile_prefix ? blockIdx.x : atomicAdd(plan.ticket, 1u);
   for (int i = tid; i < kBlockWaves * kRadix; i += kBlock)
     (&s_wave_hist[0][0])[i] = 0;
   __syncthreads();
   const u32 tile = s_tile;
   const u64 base = u64(tile) * kTile;
+  // (loaded here, before the keys' latency, not where they are used)
+  u32 digit_in = 0, prefix_in = 0;
+  if (tid < kRadix) {
+    digit_in = plan.digit_totals ? plan.digit_totals[tid]
+                                 : plan.digit_offsets[tid];
+    if (tile_prefix) prefix_in = tile_prefix[u64(tid) * gridDim.x + tile];
+  }
 
   K key[kItems];
-  u32 val[kItems], rank[kItems];
+  V val[kItems];
+  u32 rank[kItems];
   const u64 wave_base = base + u64(wave) * (kWave * kItems);
 #pragma unroll
   for (int j = 0; j < kItems; ++j) {
     const u64 idx = wave_base + u64(j) * kWave + lane;
-    const bool valid = idx < n;
-    key[j] = valid ? keys_in[idx] : ~K(0);
-    val[j] = payload(idx, valid, key[j], shift);
+    src.load(idx, idx < n, shift, key[j], val[j]);
   }
 
   // Wave-local stable ranking (item-major, then lane order == input order).
@@ -194,9 +249,9 @@ __global__ __launch_bounds__(kBlock) void onesweep_kernel(
       total += c;
     }
     // look-back: every digit owns one column of the status array
-    u64 *column = status;  // status[t * kRadix + d]
+    u64 *column = plan.status;  // status[t * kRadix + d]
     if (tile_prefix) {
-      exclusive = tile_prefix[u64(d) * gridDim.x + tile];
+      exclusive = prefix_in;
     } else if (tile == 0) {
       store_relaxed(&column[d], kFlagPrefix | total);
     } else {
@@ -218,12 +273,11 @@ __global__ __launch_bounds__(kBlock) void onesweep_kernel(
   const u32 block_start = block_exclusive_scan<kBlock>(total, s_scan);
   // the digit's start: given, or a scan of the digit totals
   u32 digit_start = 0;
-  if (tile_prefix) {
+  if (plan.digit_totals) {
     __shared__ u32 s_scan2[kBlockWaves + 1];
-    digit_start = block_exclusive_scan<kBlock>(
-        tid < kRadix ? digit_offsets[tid] : 0u, s_scan2);
-  } else if (tid < kRadix) {
-    digit_start = digit_offsets[d];
+    digit_start = block_exclusive_scan<kBlock>(digit_in, s_scan2);
+  } else {
+    digit_start = digit_in;
   }
   if (tid < kRadix) {
     s_block_start[d] = block_start;
@@ -241,7 +295,7 @@ __global__ __launch_bounds__(kBlock) void onesweep_kernel(
       s_keys[lp] = key[j];
       s_vals[lp] = val[j];
       // destination of input element idx, written in input order
-      if (dest_out) dest_out[idx] = s_global_base[dj] + lp;
+      if (plan.dest) plan.dest[idx] = s_global_base[dj] + lp;
     }
   }
   __syncthreads();
@@ -321,6 +375,34 @@ inline void clear_control(u32 *control, u64 words, hipStream_t stream,
                     256, 0, stream>>>(control, words, extra, extra_words);
 }
 
+template <bool kGated, class K, class V, class Source>
+inline void launch_shaped_pass(int block, u32 tiles, const Source &src,
+                               K *dst_k, V *dst_v, u32 n, const PassPlan &plan,
+                               hipStream_t stream) {
+  if (block == 1024)
+    onesweep_kernel<K, V, Source, 4, 1024, kGated>
+        <<<tiles, 1024, 0, stream>>>(src, dst_k, dst_v, n, plan);
+  else if (block == 512)
+    onesweep_kernel<K, V, Source, 8, 512, kGated>
+        <<<tiles, 512, 0, stream>>>(src, dst_k, dst_v, n, plan);
+  else
+    onesweep_kernel<K, V, Source, 16, 256, kGated>
+        <<<tiles, 256, 0, stream>>>(src, dst_k, dst_v, n, plan);
+}
+
+template <class K, class V, class Source>
+inline void launch_source_pass(int block, u32 tiles, const Source &src,
+                               K *dst_k, V *dst_v, u32 n, const PassPlan &plan,
+                               hipStream_t stream) {
+  if (plan.gate.value)
+    launch_shaped_pass<true>(block, tiles, src, dst_k, dst_v, n, plan, stream);
+  else
+    launch_shaped_pass<false>(block, tiles, src, dst_k, dst_v, n, plan,
+                              stream);
+}
+
+// A pass over an array of keys with 32-bit payloads.  With tile_prefix,
+// `offsets` holds the digit totals, else the digits' starts.
 template <class K, class Payload>
 inline void launch_pass(int block, u32 tiles, const K *src_k,
                         Payload payload, K *dst_k, u32 *dst_v, u32 n,
@@ -328,19 +410,71 @@ inline void launch_pass(int block, u32 tiles, const K *src_k,
                         u32 *ticket, hipStream_t stream,
                         u32 *dest = nullptr,
                         const u32 *shift_dev = nullptr,
-                        const u32 *tile_prefix = nullptr) {
-  if (block == 1024)
-    onesweep_kernel<K, Payload, 4, 1024><<<tiles, 1024, 0, stream>>>(
-        src_k, payload, dst_k, dst_v, n, shift, offsets, status, ticket,
-        dest, shift_dev, tile_prefix);
-  else if (block == 512)
-    onesweep_kernel<K, Payload, 8, 512><<<tiles, 512, 0, stream>>>(
-        src_k, payload, dst_k, dst_v, n, shift, offsets, status, ticket,
-        dest, shift_dev, tile_prefix);
-  else
-    onesweep_kernel<K, Payload, 16, 256><<<tiles, 256, 0, stream>>>(
-        src_k, payload, dst_k, dst_v, n, shift, offsets, status, ticket,
-        dest, shift_dev, tile_prefix);
+                        const u32 *tile_prefix = nullptr,
+                        const Gate &gate = Gate{},
+                        const u32 *pair = nullptr) {
+  PassPlan plan{};
+  plan.shift = shift;
+  plan.shift_dev = shift_dev;
+  plan.gate = gate;
+  plan.pair = pair;
+  (tile_prefix ? plan.digit_totals : plan.digit_offsets) = offsets;
+  plan.tile_prefix = tile_prefix;
+  plan.status = status;
+  plan.ticket = ticket;
+  plan.dest = dest;
+  launch_source_pass<K, u32>(block, tiles,
+                             ArraySource<K, Payload>{src_k, payload}, dst_k,
+                             dst_v, n, plan, stream);
+}
+
+// sort_pairs below, without its clearing launch and behind a gate.
+template <class K>
+inline hipError_t sort_pairs_cleared(const K *keys_in, u32 n, K *keys_a,
+                                     u32 *vals_a, K *keys_b, u32 *vals_b,
+                                     u32 *control, hipStream_t stream,
+                                     int block, const Gate &gate) {
+  constexpr int kPasses = passes_for<K>();
+  const int shape = block ? block : block_for(n);
+  const u32 tiles = tiles_for(n);
+  const Control c = control_layout(control, kPasses);
+  histogram_kernel<K, kPasses><<<hist_blocks_for(n), kThreads, 0, stream>>>(
+      keys_in, n, 0, c.rows, gate);
+  // behind a gate, pairs of passes over constant digits are skipped (64-bit
+  // keys of a narrow range); the first pair, which reads the input, is not
+  u32 *constant = gate.value ? c.tickets + 32 : nullptr;
+  scan_kernel<<<kPasses, kRadix, 0, stream>>>(c.rows, kPasses, c.offsets, gate,
+                                              constant, n);
+  u32 *tickets = c.tickets;
+  u64 *status = c.status;
+  const u32 *offsets = c.offsets;
+  const K *src_k = keys_in;
+  const u32 *src_v = nullptr;
+  K *dst_k = keys_b;
+  u32 *dst_v = vals_b;
+  for (int p = 0; p < kPasses; ++p) {
+    u64 *pass_status = status + u64(p) * tiles * kRadix;
+    if (p == 0) {
+      launch_pass<K>(shape, tiles, src_k, PayloadPos{}, dst_k, dst_v, n, 0,
+                     offsets, pass_status, tickets, stream, nullptr, nullptr,
+                     nullptr, gate);
+    } else {
+      launch_pass<K>(shape, tiles, src_k, PayloadIn{src_v}, dst_k, dst_v, n,
+                     8u * p, offsets + p * kRadix, pass_status, tickets + p,
+                     stream, nullptr, nullptr, nullptr, gate,
+                     constant && p >= 2 ? constant + (p & ~1) : nullptr);
+    }
+    src_k = dst_k;
+    src_v = dst_v;
+    if (dst_k == keys_b) {
+      dst_k = keys_a;
+      dst_v = vals_a;
+    } else {
+      dst_k = keys_b;
+      dst_v = vals_b;
+    }
+  }
+  return hipGetLastError();
 }
 
 // Sorts n (key, position) pairs stably.  keys_in is read only; the sorted
@@ -356,44 +490,13 @@ inline hipError_t sort_pairs(const K *keys_in, u32 n, K *keys_a, u32 *vals_a,
                              hipStream_t stream, int block = 0,
                              u64 clear_words = 0, u32 *extra = nullptr,
                              u64 extra_words = 0) {
-  constexpr int kPasses = passes_for<K>();
   if (n == 0) return hipSuccess;
-  const int shape = block ? block : block_for(n);
-  const u32 tiles = tiles_for(n);
-  const Control c = control_layout(control, kPasses);
-  clear_control(control, clear_words ? clear_words : control_words(n, kPasses),
+  clear_control(control,
+                clear_words ? clear_words
+                            : control_words(n, passes_for<K>()),
                 stream, extra, extra_words);
-  histogram_kernel<K, kPasses><<<hist_blocks_for(n), kThreads, 0, stream>>>(
-      keys_in, n, 0, c.rows);
-  scan_kernel<<<kPasses, kRadix, 0, stream>>>(c.rows, kPasses, c.offsets);
-  u32 *tickets = c.tickets;
-  u64 *status = c.status;
-  const u32 *offsets = c.offsets;
-  const K *src_k = keys_in;
-  const u32 *src_v = nullptr;
-  K *dst_k = keys_b;
-  u32 *dst_v = vals_b;
-  for (int p = 0; p < kPasses; ++p) {
-    u64 *pass_status = status + u64(p) * tiles * kRadix;
-    if (p == 0) {
-      launch_pass<K>(shape, tiles, src_k, PayloadPos{}, dst_k, dst_v, n, 0,
-                     offsets, pass_status, tickets, stream);
-    } else {
-      launch_pass<K>(shape, tiles, src_k, PayloadIn{src_v}, dst_k, dst_v, n,
-                     8u * p, offsets + p * kRadix, pass_status, tickets + p,
-                     stream);
-    }
-    src_k = dst_k;
-    src_v = dst_v;
-    if (dst_k == keys_b) {
-      dst_k = keys_a;
-      dst_v = vals_a;
-    } else {
-      dst_k = keys_b;
-      dst_v = vals_b;
-    }
-  }
-  return hipGetLastError();
+  return sort_pairs_cleared<K>(keys_in, n, keys_a, vals_a, keys_b, vals_b,
+                               control, stream, block, Gate{});
 }
 
 }  // namespace rs

@@ -114,13 +114,15 @@ static __global__ __launch_bounds__(rs::kThreads) void seg_tile_hist_kernel(
 // t] = the exclusive prefix of d's counts over the tiles and totals[d];
 // block 0 also stores the shift.  The onesweep pass then places tile t's
 // keys of digit d at (the digit's start, a scan of the totals) +
-// prefix[d * tiles + t], without a look-back.  Chunks of 4 consecutive
+// prefix[d * tiles + t], without a look-back.  *largest (nullable, zero
+// before) takes the largest total.  Chunks of 4 consecutive
 // tiles per thread, 1024 tiles per round.
 template <class K>
 static __global__ __launch_bounds__(rs::kThreads) void seg_tile_scan_kernel(
     const K *__restrict__ keys, u32 n, const u32 *__restrict__ tile_hist,
     const K *__restrict__ tile_span, u32 tiles, u32 *__restrict__ prefix,
-    u32 *__restrict__ totals, u32 *__restrict__ shift_out) {
+    u32 *__restrict__ totals, u32 *__restrict__ shift_out,
+    u32 *largest = nullptr) {
   constexpr u32 kPer = 4;
   constexpr u32 kRound = kPer * rs::kThreads;
   __shared__ u32 s_scan[rs::kThreads / kWave + 1];
@@ -201,7 +203,10 @@ static __global__ __launch_bounds__(rs::kThreads) void seg_tile_scan_kernel(
     carry += s_scan[rs::kThreads / kWave];
     __syncthreads();  // s_scan is reused by the next round
   }
-  if (threadIdx.x == 0) totals[d] = carry;
+  if (threadIdx.x == 0) {
+    totals[d] = carry;
+    if (largest && carry) atomicMax(largest, carry);
+  }
 }
 
 // Control words of a spread partition of n keys: the partition's own, the

@@ -189,7 +189,7 @@ typedef struct gd_lsm_tuning {
                                       this many keys, <= 4096 (4096)       */
   uint32_t max_runs;               /* runs kept before the smallest adjacent
                                       pair merges, 2..47 (10)              */
-  uint32_t segmented_admission;    /* 32-bit batches above 16384 keys: 1 =
+  uint32_t segmented_admission;    /* batches above small_batch_max: 1 =
                                       partition + per-segment LDS sort (1),
                                       2 = radix passes + finalize; 0 = keep */
   uint32_t merge_block;            /* merge workgroup: 256 or 512 threads
