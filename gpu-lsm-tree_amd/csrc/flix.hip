@@ -173,18 +173,20 @@ class FlixImpl : public FlixBase {
       }
       Lease<u64> begin(pool_, u64(P_) + 1);
       const u64 most = std::min<u64>(P_, n);  // touched buckets, at most
-      Lease<u32> work(pool_, most + 1);
+      Lease<u32> work(pool_, most + 2);
       const u32 *count = slices(batch, n, begin.get(), work.get(), s);
       // a wave per touched bucket, the grid sized by the upper bound (capped;
       // the waves stride over the list)
       if (S_ <= 32) {  // a half-wave per bucket
         const u64 blocks = std::min<u64>((most + 7) / 8, u64(1) << 20);
         delete_kernel<K, V, 32><<<static_cast<u32>(blocks), 256, 0, s>>>(
-            pool_view(), ring_view(), batch, begin.get(), work.get(), count);
+            pool_view(), ring_view(), batch, begin.get(), work.get(), most,
+            count);
       } else {
         const u64 blocks = std::min<u64>((most + 3) / 4, u64(1) << 20);
         delete_kernel<K, V, 64><<<static_cast<u32>(blocks), 256, 0, s>>>(
-            pool_view(), ring_view(), batch, begin.get(), work.get(), count);
+            pool_view(), ring_view(), batch, begin.get(), work.get(), most,
+            count);
       }
       GD_LAUNCH_CHECK();
     } catch (...) {
@@ -534,17 +536,18 @@ class FlixImpl : public FlixBase {
   }
 
   // Bucket slices of a sorted batch + compact list of touched buckets.
-  // Returns the device word holding the list's length (behind the list).
+  // Returns the two device words holding its counts (behind the list).
   const u32 *slices(const K *batch, u64 m, u64 *begin, u32 *work,
                     hipStream_t s) {
     bucket_slices_kernel<K><<<grid_for(u64(P_) + 1, 256), 256, 0, s>>>(
         maxv_, P_, batch, m, nullptr, begin);
     GD_LAUNCH_CHECK();
-    u32 *count = work + std::min<u64>(P_, m);
-    rs::zero_u32_kernel<<<1, 64, 0, s>>>(count, 1);
+    const u64 room = std::min<u64>(P_, m);
+    u32 *count = work + room;
+    rs::zero_u32_kernel<<<1, 64, 0, s>>>(count, 2);
     work_list_kernel<<<static_cast<u32>(
                            (u64(P_) + kWorkListBuckets - 1) / kWorkListBuckets),
-                       256, 0, s>>>(begin, P_, work, count);
+                       256, 0, s>>>(begin, P_, work, room, count);
     GD_LAUNCH_CHECK();
     return count;
   }

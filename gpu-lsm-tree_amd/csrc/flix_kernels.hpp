@@ -722,13 +722,26 @@ static __global__ void plan_reset_kernel(InsertPlan *plan) {
 
 // Removes bucket b's slice dk[pos, end) of the sorted delete batch from its
 // chain (one wave): a ballot keep-mask compacts each node, emptied non-head
-// nodes are unlinked and returned to the ring, bsize/blen follow.  dk is the
-// batch in global memory or the wave's copy of the slice in LDS (then pos =
-// 0); every search of the slice reads dk.
+// nodes are unlinked and returned to the ring together (up to kLanes of them
+// by one update of the ring's counter: its atomics, one after another from the
+// whole chip at 12 ns each, were much of a delete that empties many nodes),
+// bsize/blen follow.
+//
+// A chain's walk is a chain of memory round trips, so it is kept to one per
+// node: the next node's header and keys (the first of them ends this node's
+// share of the slice) load while this node is searched and compacted, and the
+// searches read a window of kDeleteStage slice keys in the wave's LDS (sk),
+// which moves along with the walk.  (Only a node whose share exceeds the
+// window, keys that are mostly absent, is searched in global memory.)  1.5
+// million deletes of 64-bit keys, half of them in 730 chains of 33 nodes: the
+// kernel 700 -> 327 us (368 with the long slices at their places in the list; a
+// window of 512 is no faster).
+constexpr u32 kDeleteStage = 256;
+
 template <class K, class V, u32 kLanes>
 __device__ __forceinline__ void delete_bucket(Pool<K, V> &p, Ring &ring,
                                               const K *dk, u64 pos, u64 end,
-                                              u32 b, u32 lane) {
+                                              u32 b, u32 lane, K *sk) {
   const u32 S = p.S;
   // the ballot bits of this lane's group (the wave, or its half holding
   // this bucket), lane = the slot index inside the group
@@ -737,37 +750,86 @@ __device__ __forceinline__ void delete_bucket(Pool<K, V> &p, Ring &ring,
     const u64 all = ballot(v);
     return kLanes == 64 ? all : (all >> shift) & 0xffffffffull;
   };
-  u32 node = b;
-  u32 prev = ~0u;
+  // the window: sk[0..wn) = dk[w0..w0 + wn)
+  u64 w0 = pos;
+  u32 wn = 0;
+  auto fill = [&](u64 at) {
+    // earlier searches are done before the window is written
+    __builtin_amdgcn_wave_barrier();
+    w0 = at;
+    wn = end - at < kDeleteStage ? static_cast<u32>(end - at) : kDeleteStage;
+    for (u32 j = lane; j < wn; j += kLanes) sk[j] = dk[at + j];
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  };
+  // first of sk[lo, hi) at or above key
+  auto window_bound = [&](u32 lo, u32 hi, K key) {
+    while (lo < hi) {
+      const u32 mid = (lo + hi) >> 1;
+      if (sk[mid] < key) lo = mid + 1;
+      else hi = mid;
+    }
+    return lo;
+  };
   u32 removed = 0, unlinked = 0;  // wave-uniform
+  u32 freed = 0;                  // lane i: the i-th unlinked node not yet
+                                  // returned
+  auto give_back = [&](u32 c) {
+    unsigned long long slot = 0;
+    if (lane == 0) slot = atomicAdd(ring.free_count, (unsigned long long)c);
+    slot = __shfl(slot, static_cast<int>(shift), kWave);
+    if (lane < c) ring.ids[(slot + lane) % ring.cap] = freed;
+  };
+  u32 node = b, prev = ~0u;
+  u32 nxt = p.next[node], c = p.count[node];
+  K key = lane < S ? p.keys[u64(node) * S + lane] : K(0);
+  fill(pos);
   while (true) {
-    const u32 nxt = p.next[node];
+    // the next node (every node but a head holds a key)
+    u32 n_nxt = 0, n_c = 0;
+    K n_key = K(0);
+    if (nxt) {
+      n_nxt = p.next[nxt - 1];
+      n_c = p.count[nxt - 1];
+      if (lane < S) n_key = p.keys[u64(nxt - 1) * S + lane];
+    }
+    V val = V(0);
+    if (lane < c) val = p.vals[u64(node) * S + lane];
+    if (pos == w0 + wn) fill(pos);  // (pos < end)
     // delete keys below the next node's first key (none when the slice's
     // first key is not below it)
     u64 q = end;
     if (nxt) {
-      const K first_next = p.keys[u64(nxt - 1) * S];
-      q = dk[pos] >= first_next ? pos : lower_bound_g(dk, pos, end, first_next);
+      const K first = __shfl(n_key, static_cast<int>(shift), kWave);
+      if (sk[pos - w0] >= first) {
+        q = pos;
+      } else {
+        if (w0 + wn < end && sk[wn - 1] < first && pos != w0) fill(pos);
+        q = w0 + wn < end && sk[wn - 1] < first
+                ? lower_bound_g(dk, w0 + wn, end, first)
+                : w0 + window_bound(static_cast<u32>(pos - w0), wn, first);
+      }
     }
     bool emptied = false;
     if (q > pos) {
-      const u32 c = p.count[node];
       const u64 base = u64(node) * S;
-      K key = K(0);
-      V val = V(0);
       bool hit = false;
       if (lane < c) {
-        key = p.keys[base + lane];
-        val = p.vals[base + lane];
-        const u64 f = lower_bound_g(dk, pos, q, key);
-        hit = f < q && dk[f] == key;
+        if (q <= w0 + wn) {
+          const u32 z = static_cast<u32>(q - w0);
+          const u32 f = window_bound(static_cast<u32>(pos - w0), z, key);
+          hit = f < z && sk[f] == key;
+        } else {
+          const u64 f = lower_bound_g(dk, pos, q, key);
+          hit = f < q && dk[f] == key;
+        }
       }
       const u64 keep = group_ballot(lane < c && !hit);
       const u32 kept = popc64(keep);
       if (kept != c) {
         __builtin_amdgcn_wave_barrier();
-        if ((keep >> lane) & 1ull) {
-          const u32 o = popc64(keep & ((u64(1) << lane) - 1));
+        const u32 o = popc64(keep & ((u64(1) << lane) - 1));
+        if (((keep >> lane) & 1ull) && o != lane) {  // (a slot that moves)
           p.keys[base + o] = key;
           p.vals[base + o] = val;
         }
@@ -778,20 +840,23 @@ __device__ __forceinline__ void delete_bucket(Pool<K, V> &p, Ring &ring,
     }
     pos = q;
     if (emptied) {
-      // unlink the empty non-head node and give it back to the ring
+      // unlink the empty non-head node
       if (lane == 0) {
         p.next[prev] = nxt;
         p.next[node] = 0;
-        const unsigned long long slot = atomicAdd(ring.free_count, 1ull);
-        ring.ids[slot % ring.cap] = node;
       }
-      ++unlinked;
+      if (lane == unlinked % kLanes) freed = node;
+      if (++unlinked % kLanes == 0) give_back(kLanes);
     } else {
       prev = node;
     }
     if (pos >= end || !nxt) break;
     node = nxt - 1;
+    nxt = n_nxt;
+    c = n_c;
+    key = n_key;
   }
+  if (unlinked % kLanes) give_back(unlinked % kLanes);
   if (lane == 0 && (removed || unlinked)) {
     p.bsize[b] -= removed;
     p.blen[b] -= unlinked;
@@ -802,38 +867,24 @@ __device__ __forceinline__ void delete_bucket(Pool<K, V> &p, Ring &ring,
 // non-empty slice of the sorted delete batch;
 // the waves stride over the work list, whose length the device holds (the
 // grid is sized by an upper bound, so the host reads nothing back).
-// A slice of at most kDeleteStage keys is copied to the wave's LDS first, so
-// the per-node searches of the slice (one per lane and one for the next
-// node's first key) read LDS instead of dependent global loads.
-constexpr u32 kDeleteStage = 512;
+__device__ __forceinline__ u32 work_item(const u32 *work, u64 room, u32 longs,
+                                         u32 i);
 
 template <class K, class V, u32 kLanes>
 static __global__ __launch_bounds__(256) void delete_kernel(
     Pool<K, V> p, Ring ring, const K *dk, const u64 *begin, const u32 *work,
-    const u32 *work_count) {
+    u64 room, const u32 *counts) {
   static_assert(kLanes == 32 || kLanes == 64, "a node per wave or half-wave");
   constexpr u32 kPerBlock = 256 / kLanes;  // buckets in flight per block
   __shared__ K s_dk[kPerBlock][kDeleteStage];
   const u32 lane = lane_id() % kLanes;
   const u32 w = threadIdx.x / kLanes;
-  const u32 items = *work_count;
+  const u32 longs = counts[0], items = longs + counts[1];
   for (u32 item = blockIdx.x * kPerBlock + w; item < items;
        item += gridDim.x * kPerBlock) {
-    const u32 b = work[item];
-    const u64 pos = begin[b], end = begin[b + 1];
-    const u64 m = end - pos;
-    if (m <= kDeleteStage) {
-      K *sk = s_dk[w];
-      // the previous bucket's searches are done before the slot is reused
-      __builtin_amdgcn_wave_barrier();
-      for (u32 j = lane; j < m; j += kLanes) sk[j] = dk[pos + j];
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-      delete_bucket<K, V, kLanes>(p, ring, static_cast<const K *>(sk), 0, m,
-                                  b, lane);
-    } else {
-      delete_bucket<K, V, kLanes>(p, ring, dk, pos, end, b, lane);
-    }
+    const u32 b = work_item(work, room, longs, item);
+    delete_bucket<K, V, kLanes>(p, ring, dk, begin[b], begin[b + 1], b, lane,
+                                s_dk[w]);
   }
 }
 
@@ -1200,33 +1251,56 @@ static __global__ void mark_first_kernel(const K *sk, u64 n, u32 *keep) {
     keep[i] = (i == 0 || sk[i - 1] != sk[i]) ? 1u : 0u;
 }
 
-// Buckets with a non-empty batch slice -> compact work list (in any
-// order).  A block covers kWorkListBuckets consecutive buckets, 16 per
-// thread, and takes its share of the list with one atomic, so the shared
-// counter sees one update per 4096 buckets.
+// Buckets with a non-empty batch slice -> compact work list of `room` entries
+// (in any order): those with kLongSlice keys or more from the front
+// (counts[0] of them), as their chains may be long and had better start first
+// (a delete of 1.5 million keys, 730 chains of 33 nodes: 1625 -> 1605 us with
+// its reads), the others from the back (counts[1]); see work_item.  A block covers
+// kWorkListBuckets consecutive buckets, 16 per thread, and takes its shares of
+// the list with an atomic each, so the shared counters see one update per
+// 4096 buckets.
 constexpr u32 kWorkListBuckets = 4096;
+constexpr u64 kLongSlice = 128;
 static __global__ __launch_bounds__(256) void work_list_kernel(
-    const u64 *begin, u32 buckets, u32 *work, u32 *work_count) {
+    const u64 *begin, u32 buckets, u32 *work, u64 room, u32 *counts) {
   constexpr u32 kPer = kWorkListBuckets / 256;
   __shared__ u32 s_scan[256 / kWave + 1];
-  __shared__ u32 s_base;
+  __shared__ u32 s_scan_long[256 / kWave + 1];
+  __shared__ u32 s_base, s_base_long;
   const u64 first = (u64(blockIdx.x) * 256 + threadIdx.x) * kPer;
-  u32 mask = 0, c = 0;
+  u32 mask = 0, longs = 0, c = 0, cl = 0;
 #pragma unroll
   for (u32 j = 0; j < kPer; ++j) {
     const u64 b = first + j;
-    if (b < buckets && begin[b + 1] > begin[b]) {
+    const u64 m = b < buckets ? begin[b + 1] - begin[b] : 0;
+    if (m >= kLongSlice) {
+      longs |= 1u << j;
+      ++cl;
+    } else if (m) {
       mask |= 1u << j;
       ++c;
     }
   }
   const u32 ex = block_exclusive_scan<256>(c, s_scan);
-  if (threadIdx.x == 0) s_base = atomicAdd(work_count, s_scan[256 / kWave]);
+  const u32 exl = block_exclusive_scan<256>(cl, s_scan_long);
+  if (threadIdx.x == 0) {
+    const u32 n = s_scan[256 / kWave], nl = s_scan_long[256 / kWave];
+    s_base = n ? atomicAdd(&counts[1], n) : 0u;
+    s_base_long = nl ? atomicAdd(&counts[0], nl) : 0u;
+  }
   __syncthreads();
-  u32 o = s_base + ex;
+  u32 o = s_base + ex, ol = s_base_long + exl;
 #pragma unroll
-  for (u32 j = 0; j < kPer; ++j)
-    if ((mask >> j) & 1u) work[o++] = static_cast<u32>(first + j);
+  for (u32 j = 0; j < kPer; ++j) {
+    if ((longs >> j) & 1u) work[ol++] = static_cast<u32>(first + j);
+    if ((mask >> j) & 1u) work[room - 1 - o++] = static_cast<u32>(first + j);
+  }
+}
+
+// Item i of the counts[0] + counts[1] of a work list.
+__device__ __forceinline__ u32 work_item(const u32 *work, u64 room, u32 longs,
+                                         u32 i) {
+  return i < longs ? work[i] : work[room - 1 - (i - longs)];
 }
 
 template <class K, class V>
