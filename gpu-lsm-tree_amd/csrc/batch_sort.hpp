@@ -120,18 +120,7 @@ __device__ __forceinline__ void digit_rank(typename S::Shared &sh,
     if (static_cast<u32>(j) < ipt) {
       const bool valid = wave_base + j * kWave + lane < count;
       const u32 d = static_cast<u32>(key[j] >> shift) & 0xffu;
-      u64 match = ballot(valid);
-#pragma unroll
-      for (int b = 0; b < 8; ++b) {
-        const bool bit = (d >> b) & 1u;
-        const u64 vote = ballot(bit);
-        match &= bit ? vote : ~vote;
-      }
-      u32 prior = 0;
-      if (valid) prior = lds_load(&my[d]);
-      dst[j] = prior + popc64(match & lanemask_lt());
-      if (valid && (match >> lane) == 1ull)
-        lds_store(&my[d], prior + popc64(match));
+      dst[j] = count_peers(&my[d], digit_peers(d, ballot(valid)), valid);
     }
   }
   __syncthreads();
@@ -654,14 +643,13 @@ inline hipError_t admit_batch(const typename T::K *keys, u32 n,
   lsm::seg_tile_scan_kernel<K><<<rs::kRadix, rs::kThreads, 0, s>>>(
       keys, n, c + L.hist_at, span, L.tiles, c + L.prefix_at, c + L.totals_at,
       &plan->shift_top, &plan->largest);
-  const int shape = block ? block : rs::block_for(n);
   V *vals = emit.mode == lsm::kModeErase ? nullptr : x.vals;
   rs::PassPlan top{};
   top.shift_dev = &plan->shift_top;
   top.gate = {&plan->largest, S::kCap, false};
   top.digit_totals = c + L.totals_at;
   top.tile_prefix = c + L.prefix_at;
-  rs::launch_source_pass<K, V>(shape, L.tiles, input, x.ka, vals, n, top, s);
+  rs::launch_source_pass<K, V>(rs::prefix_shape<K>(n, block), input, x.ka, vals, n, top, s);
   batch_local_kernel<S, K, V, Fn, LsmEmit<T>><<<256, S::kThreads, 0, s>>>(
       input, false, n, x.ka, vals, plan, c + L.totals_at,
       reinterpret_cast<u64 *>(c + L.status_at), emit);

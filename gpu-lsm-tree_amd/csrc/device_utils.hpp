@@ -54,6 +54,48 @@ __device__ __forceinline__ void lds_store(u32 *p, u32 v) {
                      __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
+// The lanes of the wave (of `among`) that hold the same 8-bit digit as this
+// one: how many there are, and how many of them are lower lanes.  Called by
+// the whole wave; lanes outside `among` get nothing of use.
+//
+// Eight ballots, four instructions a bit: the lane's bit widened to a mask, the
+// ballot, and one three-operand logic instruction per half of the peers' mask
+// (the plain select between a ballot and its complement compiled to eleven, a
+// third of a radix pass's instructions).
+struct DigitPeers {
+  u32 before, count;
+  // the highest lane of the group
+  __device__ __forceinline__ bool last() const { return before + 1 == count; }
+};
+__device__ __forceinline__ DigitPeers digit_peers(u32 digit,
+                                                  u64 among = ~0ull) {
+  u32 lo = static_cast<u32>(among), hi = static_cast<u32>(among >> 32);
+#pragma unroll
+  for (int b = 0; b < 8; ++b) {
+    u32 mine = __builtin_amdgcn_sbfe(digit, b, 1);
+    asm("" : "+v"(mine));  // (else the ballot tests a shifted copy of its own)
+    const u64 vote = ballot(mine != 0);
+    // peers & ~(mine ^ vote)
+    lo = __builtin_amdgcn_bitop3_b32(lo, mine, static_cast<u32>(vote), 0x90);
+    hi = __builtin_amdgcn_bitop3_b32(hi, mine, static_cast<u32>(vote >> 32),
+                                     0x90);
+  }
+  return {__builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0)),
+          static_cast<u32>(__builtin_popcount(lo) + __builtin_popcount(hi))};
+}
+// Counts the digit's peers at *counter (this wave's own LDS counter of the
+// digit) and returns how many of the digit came before this lane: the group's
+// last lane adds, then all read.  A wave's LDS operations execute in program
+// order, so the calls of several items wait for nothing in between.
+__device__ __forceinline__ u32 count_peers(u32 *counter, const DigitPeers &g,
+                                           bool valid = true) {
+  if (valid && g.last())
+    __hip_atomic_fetch_add((lds_u32 *)(counter), g.count, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_WORKGROUP);
+  __builtin_amdgcn_wave_barrier();
+  return lds_load(counter) - g.count + g.before;
+}
+
 // Wave-wide inclusive scan of a u32 through DPP-backed shuffles.
 __device__ __forceinline__ u32 wave_inclusive_scan(u32 v) {
   const u32 lane = lane_id();

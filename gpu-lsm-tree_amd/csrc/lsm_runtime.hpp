@@ -1185,8 +1185,7 @@ class LsmT : public HandleBase {
           keys, n, tile_hist.get(), span, tiles, tile_prefix, pc.offsets,
           c + L.shift_at);
       rs::launch_pass<u32>(
-          tuning_.sort_block ? tuning_.sort_block : rs::block_for(n), tiles,
-          keys, SegPayload{values, flags, mode}, ka.get(), va.get(), n, 0,
+          rs::prefix_shape<K>(n, tuning_.sort_block), keys, SegPayload{values, flags, mode}, ka.get(), va.get(), n, 0,
           pc.offsets, pc.status, pc.tickets, s, nullptr, c + L.shift_at,
           tile_prefix);
     }

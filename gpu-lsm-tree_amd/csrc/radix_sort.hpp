@@ -163,6 +163,16 @@ struct PassPlan {
   u32 *dest;               // nullable: each input element's place
 };
 
+// Workgroups go to the 8 XCDs in turn: workgroup i's tile, such that each XCD
+// takes consecutive tiles.
+__device__ __forceinline__ u32 xcd_tile(u32 i, u32 tiles) {
+  const u32 x = i % 8, each = tiles / 8, more = tiles % 8;
+  return x * each + (x < more ? x : more) + i / 8;
+}
+
+// Tiles that a look-back reads at once.
+constexpr u32 kLookBack = 4;
+
 // kBlock threads x kItems keys per tile; threads below 256 own one digit each
 // for the per-digit bookkeeping.
 template <class K, class V, class Source, int kItems, int kBlock, bool kGated>
@@ -181,7 +191,6 @@ __global__ __launch_bounds__(kBlock) void onesweep_kernel(
   constexpr int kBlockWaves = kBlock / kWave;
   __shared__ u32 s_tile;
   __shared__ u32 s_wave_hist[kBlockWaves][kRadix];
-  __shared__ u32 s_block_start[kRadix];
   __shared__ u32 s_global_base[kRadix];
   __shared__ u32 s_scan[kBlockWaves + 1];
   __shared__ K s_keys[kTile];
@@ -190,12 +199,14 @@ __global__ __launch_bounds__(kBlock) void onesweep_kernel(
   const u32 tid = threadIdx.x;
   const u32 lane = lane_id();
   const u32 wave = tid / kWave;
-  if (tid == 0) s_tile = tile_prefix ? blockIdx.x : atomicAdd(plan.ticket, 1u);
+  if (tid == 0) s_tile = tile_prefix ? xcd_tile(blockIdx.x, gridDim.x)
+                                   : atomicAdd(plan.ticket, 1u);
   for (int i = tid; i < kBlockWaves * kRadix; i += kBlock)
     (&s_wave_hist[0][0])[i] = 0;
   __syncthreads();
   const u32 tile = s_tile;
-  const u64 base = u64(tile) * kTile;
+  const u32 base = tile * kTile;  // (below n, so nothing here overflows)
+  const u32 count = n - base < u32(kTile) ? n - base : u32(kTile);
   // (loaded here, before the keys' latency, not where they are used)
   u32 digit_in = 0, prefix_in = 0;
   if (tid < kRadix) {
@@ -204,49 +215,37 @@ __global__ __launch_bounds__(kBlock) void onesweep_kernel(
     if (tile_prefix) prefix_in = tile_prefix[u64(tid) * gridDim.x + tile];
   }
 
+  // Places behind the input's end hold a key of the highest digit: they rank
+  // behind every key of the tile and are not written.
   K key[kItems];
   V val[kItems];
   u32 rank[kItems];
-  const u64 wave_base = base + u64(wave) * (kWave * kItems);
+  const u32 wave_at = wave * (kWave * kItems) + lane;
 #pragma unroll
   for (int j = 0; j < kItems; ++j) {
-    const u64 idx = wave_base + u64(j) * kWave + lane;
-    src.load(idx, idx < n, shift, key[j], val[j]);
+    const u32 i = wave_at + j * kWave;
+    src.load(base + i, i < count, shift, key[j], val[j]);
   }
 
   // Wave-local stable ranking (item-major, then lane order == input order).
   u32 *my_hist = s_wave_hist[wave];
 #pragma unroll
   for (int j = 0; j < kItems; ++j) {
-    const u64 idx = wave_base + u64(j) * kWave + lane;
-    const bool valid = idx < n;
     const u32 d = static_cast<u32>(key[j] >> shift) & 0xffu;
-    u64 match = ballot(valid);
-#pragma unroll
-    for (int b = 0; b < 8; ++b) {
-      const bool bit = (d >> b) & 1u;
-      const u64 vote = ballot(bit);
-      match &= bit ? vote : ~vote;
-    }
-    u32 prior = 0;
-    if (valid) prior = lds_load(&my_hist[d]);
-    rank[j] = prior + popc64(match & lanemask_lt());
-    // the highest lane of each digit group advances the counter
-    if (valid && (match >> lane) == 1ull)
-      lds_store(&my_hist[d], prior + popc64(match));
+    rank[j] = count_peers(&my_hist[d], digit_peers(d));
   }
   __syncthreads();
 
   // Per digit: wave prefixes, tile total, global base via look-back.
   const u32 d = tid;
   u32 total = 0;
+  u32 wave_start[kBlockWaves];
   u64 exclusive = 0;
   if (tid < kRadix) {
 #pragma unroll
     for (int w = 0; w < kBlockWaves; ++w) {
-      const u32 c = s_wave_hist[w][d];
-      s_wave_hist[w][d] = total;
-      total += c;
+      wave_start[w] = total;
+      total += s_wave_hist[w][d];
     }
     // look-back: every digit owns one column of the status array
     u64 *column = plan.status;  // status[t * kRadix + d]
@@ -256,15 +255,27 @@ __global__ __launch_bounds__(kBlock) void onesweep_kernel(
       store_relaxed(&column[d], kFlagPrefix | total);
     } else {
       store_relaxed(&column[u64(tile) * kRadix + d], kFlagAggregate | total);
-      long long t = static_cast<long long>(tile) - 1;
-      while (true) {
-        u64 word;
-        do {
-          word = load_relaxed(&column[u64(t) * kRadix + d]);
-        } while ((word >> kFlagShift) == 0);
-        exclusive += word & kValueMask;
-        if (word & kFlagPrefix) break;
-        --t;
+      u32 t = tile;  // the tiles from t on are summed
+      bool open = true;
+      while (open) {
+        u64 word[kLookBack];
+#pragma unroll
+        for (u32 q = 0; q < kLookBack; ++q)
+          word[q] = q < t ? load_relaxed(&column[u64(t - 1 - q) * kRadix + d])
+                          : kFlagPrefix;
+        u32 ready = 0;
+        bool next = true;  // every word so far was there, none a prefix
+#pragma unroll
+        for (u32 q = 0; q < kLookBack; ++q) {
+          next = next && (word[q] >> kFlagShift) != 0;
+          if (next) {
+            exclusive += word[q] & kValueMask;
+            ++ready;
+            if (word[q] & kFlagPrefix) next = open = false;
+          }
+        }
+        t = ready < t ? t - ready : 0;
+        if (ready == 0) __builtin_amdgcn_s_sleep(4);
       }
       store_relaxed(&column[u64(tile) * kRadix + d],
                     kFlagPrefix | (exclusive + total));
@@ -280,7 +291,9 @@ __global__ __launch_bounds__(kBlock) void onesweep_kernel(
     digit_start = digit_in;
   }
   if (tid < kRadix) {
-    s_block_start[d] = block_start;
+#pragma unroll
+    for (int w = 0; w < kBlockWaves; ++w)
+      s_wave_hist[w][d] = block_start + wave_start[w];
     s_global_base[d] = digit_start + static_cast<u32>(exclusive) - block_start;
   }
   __syncthreads();
@@ -288,26 +301,36 @@ __global__ __launch_bounds__(kBlock) void onesweep_kernel(
   // Scatter into LDS in digit order.
 #pragma unroll
   for (int j = 0; j < kItems; ++j) {
-    const u64 idx = wave_base + u64(j) * kWave + lane;
-    if (idx < n) {
+    const u32 dj = static_cast<u32>(key[j] >> shift) & 0xffu;
+    rank[j] += my_hist[dj];
+    s_keys[rank[j]] = key[j];
+    s_vals[rank[j]] = val[j];
+  }
+  // destination of each input element, written in input order
+  if (plan.dest) {
+#pragma unroll
+    for (int j = 0; j < kItems; ++j) {
+      const u32 i = wave_at + j * kWave;
       const u32 dj = static_cast<u32>(key[j] >> shift) & 0xffu;
-      const u32 lp = s_block_start[dj] + s_wave_hist[wave][dj] + rank[j];
-      s_keys[lp] = key[j];
-      s_vals[lp] = val[j];
-      // destination of input element idx, written in input order
-      if (plan.dest) plan.dest[idx] = s_global_base[dj] + lp;
+      if (i < count) plan.dest[base + i] = s_global_base[dj] + rank[j];
     }
   }
   __syncthreads();
 
-  const u32 count =
-      base >= n ? 0u : static_cast<u32>(n - base < u64(kTile) ? n - base
-                                                              : u64(kTile));
-  for (u32 i = tid; i < count; i += kBlock) {
-    const K k = s_keys[i];
-    const u32 pos = s_global_base[static_cast<u32>(k >> shift) & 0xffu] + i;
-    keys_out[pos] = k;
-    if (vals_out) vals_out[pos] = s_vals[i];
+  // all LDS reads before the stores
+#pragma unroll
+  for (int j = 0; j < kItems; ++j) {
+    const u32 i = j * kBlock + tid;
+    key[j] = s_keys[i];
+    val[j] = s_vals[i];
+    rank[j] = s_global_base[static_cast<u32>(key[j] >> shift) & 0xffu] + i;
+  }
+#pragma unroll
+  for (int j = 0; j < kItems; ++j) {
+    if (j * kBlock + tid < count) {
+      keys_out[rank[j]] = key[j];
+      if (vals_out) vals_out[rank[j]] = val[j];
+    }
   }
 }
 
@@ -328,15 +351,37 @@ static __global__ void zero_u32_kernel(u32 *p, u64 n) {
 }
 
 
-// Tile = 4096 keys: 1024 threads x 4 keys below 2^22 keys (the 256-tile
-// passes of 2^20-key batches run one tile per CU, so more waves per tile
-// hide more latency), 256 x 16 above.  (2048-key tiles were measured
-// slower on MI355X: more look-back steps.)
-inline int block_for(u64 n) { return n < (u64(1) << 22) ? 1024 : 256; }
+// A pass's workgroups: `block` threads with `items` keys each, a tile per
+// workgroup.
+struct PassShape {
+  int block, items;
+  u32 tiles;
+};
 
 inline u32 tiles_for(u64 n) {
   const u64 tile = 4096;
   return static_cast<u32>((n + tile - 1) / tile);
+}
+
+// Passes over tiles of 4096 keys whose digit prefixes are known: a tile per CU
+// wants many waves (up to 2^20 keys), several tiles a CU want several
+// workgroups (3,000,017 32-bit keys: 20.6 us in workgroups of 1024, 17.0 of
+// 512, 14.9 of 256; 64-bit keys 22.1, 18.9 and 20.4).  block != 0: as told.
+template <class K>
+inline PassShape prefix_shape(u64 n, int block = 0) {
+  const int b = block ? block
+                : n <= (u64(1) << 20) ? 1024 : sizeof(K) == 8 ? 512 : 256;
+  return {b, 4096 / b, tiles_for(n)};
+}
+
+// Passes whose tiles chain their offsets: the chain costs some 15 ns a tile,
+// half of a pass's time, so the tiles are 8192 keys where they still fill the
+// chip (8,388,608 32-bit keys: 73 us with tiles of 4096, 61 so; 1,500,003
+// 64-bit keys: 27 and 21; 300,000: 13.7 and 15.5).
+inline PassShape chained_shape(u64 n, int block = 0) {
+  if (block) return {block, 4096 / block, tiles_for(n)};
+  if (n < 600000) return {1024, 4, tiles_for(n)};
+  return {1024, 8, static_cast<u32>((n + 8191) / 8192)};
 }
 
 // Workspace (u32 words) of a sort of n keys in `passes` digit passes, not
@@ -376,35 +421,39 @@ inline void clear_control(u32 *control, u64 words, hipStream_t stream,
 }
 
 template <bool kGated, class K, class V, class Source>
-inline void launch_shaped_pass(int block, u32 tiles, const Source &src,
-                               K *dst_k, V *dst_v, u32 n, const PassPlan &plan,
+inline void launch_shaped_pass(const PassShape &h, const Source &src, K *dst_k,
+                               V *dst_v, u32 n, const PassPlan &plan,
                                hipStream_t stream) {
-  if (block == 1024)
+  if (h.block == 1024 && h.items == 8) {
+    if constexpr (sizeof(K) + sizeof(V) <= 12)  // (within the LDS)
+      onesweep_kernel<K, V, Source, 8, 1024, kGated>
+          <<<h.tiles, 1024, 0, stream>>>(src, dst_k, dst_v, n, plan);
+  } else if (h.block == 1024) {
     onesweep_kernel<K, V, Source, 4, 1024, kGated>
-        <<<tiles, 1024, 0, stream>>>(src, dst_k, dst_v, n, plan);
-  else if (block == 512)
+        <<<h.tiles, 1024, 0, stream>>>(src, dst_k, dst_v, n, plan);
+  } else if (h.block == 512) {
     onesweep_kernel<K, V, Source, 8, 512, kGated>
-        <<<tiles, 512, 0, stream>>>(src, dst_k, dst_v, n, plan);
-  else
+        <<<h.tiles, 512, 0, stream>>>(src, dst_k, dst_v, n, plan);
+  } else {
     onesweep_kernel<K, V, Source, 16, 256, kGated>
-        <<<tiles, 256, 0, stream>>>(src, dst_k, dst_v, n, plan);
+        <<<h.tiles, 256, 0, stream>>>(src, dst_k, dst_v, n, plan);
+  }
 }
 
 template <class K, class V, class Source>
-inline void launch_source_pass(int block, u32 tiles, const Source &src,
+inline void launch_source_pass(const PassShape &shape, const Source &src,
                                K *dst_k, V *dst_v, u32 n, const PassPlan &plan,
                                hipStream_t stream) {
   if (plan.gate.value)
-    launch_shaped_pass<true>(block, tiles, src, dst_k, dst_v, n, plan, stream);
+    launch_shaped_pass<true>(shape, src, dst_k, dst_v, n, plan, stream);
   else
-    launch_shaped_pass<false>(block, tiles, src, dst_k, dst_v, n, plan,
-                              stream);
+    launch_shaped_pass<false>(shape, src, dst_k, dst_v, n, plan, stream);
 }
 
 // A pass over an array of keys with 32-bit payloads.  With tile_prefix,
 // `offsets` holds the digit totals, else the digits' starts.
 template <class K, class Payload>
-inline void launch_pass(int block, u32 tiles, const K *src_k,
+inline void launch_pass(const PassShape &shape, const K *src_k,
                         Payload payload, K *dst_k, u32 *dst_v, u32 n,
                         u32 shift, const u32 *offsets, u64 *status,
                         u32 *ticket, hipStream_t stream,
@@ -423,7 +472,7 @@ inline void launch_pass(int block, u32 tiles, const K *src_k,
   plan.status = status;
   plan.ticket = ticket;
   plan.dest = dest;
-  launch_source_pass<K, u32>(block, tiles,
+  launch_source_pass<K, u32>(shape,
                              ArraySource<K, Payload>{src_k, payload}, dst_k,
                              dst_v, n, plan, stream);
 }
@@ -435,8 +484,7 @@ inline hipError_t sort_pairs_cleared(const K *keys_in, u32 n, K *keys_a,
                                      u32 *control, hipStream_t stream,
                                      int block, const Gate &gate) {
   constexpr int kPasses = passes_for<K>();
-  const int shape = block ? block : block_for(n);
-  const u32 tiles = tiles_for(n);
+  const PassShape shape = chained_shape(n, block);
   const Control c = control_layout(control, kPasses);
   histogram_kernel<K, kPasses><<<hist_blocks_for(n), kThreads, 0, stream>>>(
       keys_in, n, 0, c.rows, gate);
@@ -453,13 +501,13 @@ inline hipError_t sort_pairs_cleared(const K *keys_in, u32 n, K *keys_a,
   K *dst_k = keys_b;
   u32 *dst_v = vals_b;
   for (int p = 0; p < kPasses; ++p) {
-    u64 *pass_status = status + u64(p) * tiles * kRadix;
+    u64 *pass_status = status + u64(p) * tiles_for(n) * kRadix;
     if (p == 0) {
-      launch_pass<K>(shape, tiles, src_k, PayloadPos{}, dst_k, dst_v, n, 0,
+      launch_pass<K>(shape, src_k, PayloadPos{}, dst_k, dst_v, n, 0,
                      offsets, pass_status, tickets, stream, nullptr, nullptr,
                      nullptr, gate);
     } else {
-      launch_pass<K>(shape, tiles, src_k, PayloadIn{src_v}, dst_k, dst_v, n,
+      launch_pass<K>(shape, src_k, PayloadIn{src_v}, dst_k, dst_v, n,
                      8u * p, offsets + p * kRadix, pass_status, tickets + p,
                      stream, nullptr, nullptr, nullptr, gate,
                      constant && p >= 2 ? constant + (p & ~1) : nullptr);

@@ -261,10 +261,9 @@ inline void partition_by_spread(const K *keys, u32 n, K *keys_out,
   spread_counts<K>(keys, n, control, s, extra, extra_words);
   const SpreadLayout<K> L(n);
   const rs::Control pc = rs::control_layout(control, 1);
-  const u32 tiles = rs::tiles_for(n);
-  const u32 *tile_prefix =
-      reinterpret_cast<u32 *>(pc.status) + u64(tiles) * rs::kRadix;
-  rs::launch_pass<K>(block ? block : rs::block_for(n), tiles, keys, payload,
+  const u32 *tile_prefix = reinterpret_cast<u32 *>(pc.status) +
+                           u64(rs::tiles_for(n)) * rs::kRadix;
+  rs::launch_pass<K>(rs::prefix_shape<K>(n, block), keys, payload,
                      keys_out, pos_out, n, 0, pc.offsets, pc.status,
                      pc.tickets, s, dest, control + L.shift_at,
                      tile_prefix);
@@ -358,18 +357,7 @@ __device__ __forceinline__ void seg_rank(SegShared &sh, u32 (*hist)[256],
     if (static_cast<u32>(j) < ipt) {
       const bool valid = wave_base + j * kWave + lane < count;
       const u32 d = (key[j] >> shift) & 0xffu;
-      u64 match = ballot(valid);
-#pragma unroll
-      for (int b = 0; b < 8; ++b) {
-        const bool bit = (d >> b) & 1u;
-        const u64 vote = ballot(bit);
-        match &= bit ? vote : ~vote;
-      }
-      u32 prior = 0;
-      if (valid) prior = lds_load(&my_hist[d]);
-      rank[j] = prior + popc64(match & lanemask_lt());
-      if (valid && (match >> lane) == 1ull)
-        lds_store(&my_hist[d], prior + popc64(match));
+      rank[j] = count_peers(&my_hist[d], digit_peers(d, ballot(valid)), valid);
     }
   }
   __syncthreads();
