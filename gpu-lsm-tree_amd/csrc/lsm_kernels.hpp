@@ -250,7 +250,9 @@ enum FinalizeMode : int {
 // with tombstones set the tombstone flag.  The radix directory (dir_bits
 // bits) is written here too: sorted position i owns the directory entries
 // of the buckets in (bucket(key[i-1]), bucket(key[i])] and writes them the
-// number of survivors before position i (the output row of its key).
+// number of survivors before position i (the output row of its key).  sp: the
+// sorted updates' positions or, where values is null, the values themselves
+// (inserts of 32-bit values).
 template <class T>
 __global__ __launch_bounds__(kFinThreads) void finalize_batch_kernel(
     const typename T::K *__restrict__ sk, const u32 *__restrict__ sp, u32 n,
@@ -310,20 +312,34 @@ __global__ __launch_bounds__(kFinThreads) void finalize_batch_kernel(
   __syncthreads();
   const u64 out_base = s_base;
   u32 low = 0, tombs = 0;
+  // (a surviving row's loads; all are issued before the first is waited for)
+  V val[kFinItems];
+  u32 tomb = 0;
+#pragma unroll
+  for (int j = 0; j < kFinItems; ++j) {
+    const bool kept = (mask[j] >> lane) & 1ull;
+    val[j] = kept ? V(sp[base + u64(j) * kFinThreads + threadIdx.x]) : V(0);
+  }
+  if (mode == kModeErase) {
+    tomb = ~0u;
+  } else if (values) {
+#pragma unroll
+    for (int j = 0; j < kFinItems; ++j) {
+      if (!((mask[j] >> lane) & 1ull)) continue;
+      const u32 p = static_cast<u32>(val[j]);
+      if (mode == kModeMixed && erase_flags[p] != 0) tomb |= 1u << j;
+      val[j] = values[p];
+    }
+  }
 #pragma unroll
   for (int j = 0; j < kFinItems; ++j) {
     if (!((mask[j] >> lane) & 1ull)) continue;
-    const u64 i = base + u64(j) * kFinThreads + threadIdx.x;
     const u64 o = out_base + s_off[j][wave] + popc64(mask[j] & lanemask_lt());
-    const u32 p = sp[i];
-    bool tomb;
-    if (mode == kModeErase) tomb = true;
-    else if (mode == kModeMixed) tomb = erase_flags[p] != 0;
-    else tomb = false;
-    const V v = tomb ? V(0) : values[p];
-    out[o] = T::make((key[j] & T::kLow) | (tomb ? T::kTomb : K(0)), v);
+    const bool dead = (tomb >> j) & 1u;
+    out[o] = T::make((key[j] & T::kLow) | (dead ? T::kTomb : K(0)),
+                     dead ? V(0) : val[j]);
     low += key[j] < T::kTomb;
-    tombs += tomb;
+    tombs += dead;
   }
   // directory entries inside the bucket window
   const u32 shift = T::kBits - dir_bits;

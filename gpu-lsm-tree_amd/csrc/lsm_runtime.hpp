@@ -1087,7 +1087,12 @@ class LsmT : public HandleBase {
     GD_LAUNCH_CHECK();
   }
 
-  // Sorts one tile of updates into a new run.
+  // Sorts one tile of updates into a new run.  32-bit builds above
+  // kSegmentedMax take the radix passes: their segments do not fit the LDS (a
+  // workgroup would sort each in memory).  2,500,000 uniform keys: 298 us by
+  // segments, 197 by passes; 15,000,001: 919 and 631.  (Keys that come twice
+  // each, whose segments are deduplicated first: 4,000,000 220 and 240.)
+  static constexpr u32 kSegmentedMax = u32(1) << 21;
   Run sorted_run(const K *keys, const V *values, const u8 *flags, u32 n,
                  int mode, hipStream_t s) {
     Run r = alloc_run(n);
@@ -1101,7 +1106,8 @@ class LsmT : public HandleBase {
     }
     if (tuning_.segmented_admission == 1) {
       if constexpr (sizeof(K) == 4) {
-        if (n > 16384) return segmented_run(keys, values, flags, n, mode, s, r);
+        if (n > 16384 && n <= kSegmentedMax)
+          return segmented_run(keys, values, flags, n, mode, s, r);
       }
       // (a larger build's digits would not fit the LDS)
       if (n <= kMaximumOperationTile)
@@ -1112,6 +1118,12 @@ class LsmT : public HandleBase {
     const u64 fin_words = 64 + 2ull * fin_tiles;  // ticket pad + status u64
     Lease<K> ka(pool_, n), kb(pool_, n);
     Lease<u32> va(pool_, n), vb(pool_, n);
+    // 32-bit values of inserts ride along; else the positions do, and values
+    // and flags are gathered
+    const u32 *carried = nullptr;
+    if constexpr (sizeof(V) == 4) {
+      if (mode == kModeInsert) carried = values;
+    }
     Lease<u32> ctrl(pool_, sort_words + fin_words);
     u32 *fin_ctrl = ctrl.get() + sort_words;
     // the sort's clearing launch also clears the finalize state behind its
@@ -1119,9 +1131,10 @@ class LsmT : public HandleBase {
     GD_HIP(rs::sort_pairs<K>(keys, n, ka.get(), va.get(), kb.get(), vb.get(),
                              ctrl.get(), s, tuning_.sort_block,
                              sort_words + fin_words,
-                             reinterpret_cast<u32 *>(r.meta()), kMetaWords));
+                             reinterpret_cast<u32 *>(r.meta()), kMetaWords,
+                             carried));
     finalize_batch_kernel<T><<<fin_tiles, kFinThreads, 0, s>>>(
-        ka.get(), va.get(), n, values, flags, mode, r.rows, r.meta(),
+        ka.get(), va.get(), n, carried ? nullptr : values, flags, mode, r.rows, r.meta(),
         r.entries(), r.max_bits, reinterpret_cast<u64 *>(fin_ctrl + 64),
         fin_ctrl, rs::Gate{});
     GD_LAUNCH_CHECK();

@@ -444,7 +444,7 @@ template <class K, class V, class Source>
 inline void launch_source_pass(const PassShape &shape, const Source &src,
                                K *dst_k, V *dst_v, u32 n, const PassPlan &plan,
                                hipStream_t stream) {
-  if (plan.gate.value)
+  if (plan.gate.value || plan.pair)
     launch_shaped_pass<true>(shape, src, dst_k, dst_v, n, plan, stream);
   else
     launch_shaped_pass<false>(shape, src, dst_k, dst_v, n, plan, stream);
@@ -482,27 +482,28 @@ template <class K>
 inline hipError_t sort_pairs_cleared(const K *keys_in, u32 n, K *keys_a,
                                      u32 *vals_a, K *keys_b, u32 *vals_b,
                                      u32 *control, hipStream_t stream,
-                                     int block, const Gate &gate) {
+                                     int block, const Gate &gate,
+                                     const u32 *vals_in = nullptr) {
   constexpr int kPasses = passes_for<K>();
   const PassShape shape = chained_shape(n, block);
   const Control c = control_layout(control, kPasses);
   histogram_kernel<K, kPasses><<<hist_blocks_for(n), kThreads, 0, stream>>>(
       keys_in, n, 0, c.rows, gate);
-  // behind a gate, pairs of passes over constant digits are skipped (64-bit
-  // keys of a narrow range); the first pair, which reads the input, is not
-  u32 *constant = gate.value ? c.tickets + 32 : nullptr;
+  // pairs of passes over constant digits are skipped (64-bit keys of a narrow
+  // range); the first pair, which reads the input, is not
+  u32 *constant = gate.value || kPasses > 4 ? c.tickets + 32 : nullptr;
   scan_kernel<<<kPasses, kRadix, 0, stream>>>(c.rows, kPasses, c.offsets, gate,
                                               constant, n);
   u32 *tickets = c.tickets;
   u64 *status = c.status;
   const u32 *offsets = c.offsets;
   const K *src_k = keys_in;
-  const u32 *src_v = nullptr;
+  const u32 *src_v = vals_in;
   K *dst_k = keys_b;
   u32 *dst_v = vals_b;
   for (int p = 0; p < kPasses; ++p) {
     u64 *pass_status = status + u64(p) * tiles_for(n) * kRadix;
-    if (p == 0) {
+    if (p == 0 && !vals_in) {
       launch_pass<K>(shape, src_k, PayloadPos{}, dst_k, dst_v, n, 0,
                      offsets, pass_status, tickets, stream, nullptr, nullptr,
                      nullptr, gate);
@@ -531,20 +532,22 @@ inline hipError_t sort_pairs_cleared(const K *keys_in, u32 n, K *keys_a,
 // words.  All launches go to `stream`.
 // clear_words (0 = control_words(n, passes)) words of `control` and
 // extra[0..extra_words) are cleared by the first launch, so callers can
-// place zero-initialised state of their own behind the sort's.
+// place zero-initialised state of their own behind the sort's.  vals_in
+// (nullable): payloads to carry instead of the positions.
 template <class K>
 inline hipError_t sort_pairs(const K *keys_in, u32 n, K *keys_a, u32 *vals_a,
                              K *keys_b, u32 *vals_b, u32 *control,
                              hipStream_t stream, int block = 0,
                              u64 clear_words = 0, u32 *extra = nullptr,
-                             u64 extra_words = 0) {
+                             u64 extra_words = 0,
+                             const u32 *vals_in = nullptr) {
   if (n == 0) return hipSuccess;
   clear_control(control,
                 clear_words ? clear_words
                             : control_words(n, passes_for<K>()),
                 stream, extra, extra_words);
   return sort_pairs_cleared<K>(keys_in, n, keys_a, vals_a, keys_b, vals_b,
-                               control, stream, block, Gate{});
+                               control, stream, block, Gate{}, vals_in);
 }
 
 }  // namespace rs
