@@ -387,18 +387,18 @@ class LsmT : public HandleBase {
     u64 count = 0;
     try {
       if (!runs_.empty()) {
-        Run merged = merge_all(runs_, /*consume=*/false, s);
-        count = read_count(merged, s);
+        Live live = live_rows(s);
+        count = live.count;
         if (count <= capacity && count) {
           if (!out_keys || !out_vals) {
-            free_run(merged);
+            if (live.merged) free_run(live.run);
             throw Error(GD_INVALID_ARGUMENT, "null dump output");
           }
           decode_run_kernel<T><<<grid_for(count, 256, 1u << 16), 256, 0, s>>>(
-              merged.rows, merged.meta(), out_keys, out_vals);
+              live.run.rows, live.run.meta(), out_keys, out_vals);
           GD_LAUNCH_CHECK();
         }
-        free_run(merged);
+        if (live.merged) free_run(live.run);
         GD_HIP(hipStreamSynchronize(s));
       }
     } catch (...) {
@@ -441,20 +441,18 @@ class LsmT : public HandleBase {
     if (!path) throw Error(GD_INVALID_ARGUMENT, "null snapshot path");
     order_.begin(s);
     u64 count = 0;
-    // the merged copy goes back to the pool on every exit path
-    Run merged{};
-    bool have = false;
+    // a merged copy goes back to the pool on every exit path
+    Live live{};
     try {
       if (!runs_.empty()) {
-        merged = merge_all(runs_, /*consume=*/false, s);
-        have = true;
-        count = read_count(merged, s);
+        live = live_rows(s);
+        count = live.count;
       }
       Lease<K> k(pool_, std::max<u64>(count, 1));
       Lease<V> v(pool_, std::max<u64>(count, 1));
       if (count) {
         decode_run_kernel<T><<<grid_for(count, 256, 1u << 16), 256, 0, s>>>(
-            merged.rows, merged.meta(), k.get(), v.get());
+            live.run.rows, live.run.meta(), k.get(), v.get());
         GD_LAUNCH_CHECK();
       }
       FileCloser f(std::fopen(path, "wb"));
@@ -475,10 +473,10 @@ class LsmT : public HandleBase {
       write_all(f.p, &h, sizeof(h));
       // a failed final flush (a full disk) must not report success
       f.close_checked();
-      if (have) free_run(merged);
-      have = false;
+      if (live.merged) free_run(live.run);
+      live.merged = false;
     } catch (...) {
-      if (have) free_run(merged);
+      if (live.merged) free_run(live.run);
       order_.end(s);
       throw;
     }
@@ -1118,14 +1116,14 @@ class LsmT : public HandleBase {
     const u64 fin_words = 64 + 2ull * fin_tiles;  // ticket pad + status u64
     Lease<K> ka(pool_, n), kb(pool_, n);
     Lease<u32> va(pool_, n), vb(pool_, n);
+    Lease<u32> ctrl(pool_, sort_words + fin_words);
+    u32 *fin_ctrl = ctrl.get() + sort_words;
     // 32-bit values of inserts ride along; else the positions do, and values
     // and flags are gathered
     const u32 *carried = nullptr;
     if constexpr (sizeof(V) == 4) {
       if (mode == kModeInsert) carried = values;
     }
-    Lease<u32> ctrl(pool_, sort_words + fin_words);
-    u32 *fin_ctrl = ctrl.get() + sort_words;
     // the sort's clearing launch also clears the finalize state behind its
     // own and the run header
     GD_HIP(rs::sort_pairs<K>(keys, n, ka.get(), va.get(), kb.get(), vb.get(),
@@ -1415,11 +1413,29 @@ class LsmT : public HandleBase {
     }
   }
 
-  u32 read_count(const Run &r, hipStream_t s) {
+  RunMeta read_meta(const Run &r, hipStream_t s) {
     RunMeta m{};
     GD_HIP(hipMemcpyAsync(&m, r.meta(), sizeof(m), hipMemcpyDeviceToHost, s));
     GD_HIP(hipStreamSynchronize(s));
-    return m.count;
+    return m;
+  }
+  u32 read_count(const Run &r, hipStream_t s) { return read_meta(r, s).count; }
+
+  // The live rows as one run: the only run where it holds no tombstones (as a
+  // bulk build leaves it: merging it with an empty run took 89 of a 15,000,001
+  // row dump's 130 us), else a merged copy, which the caller frees.
+  struct Live {
+    Run run;
+    u64 count;
+    bool merged;
+  };
+  Live live_rows(hipStream_t s) {
+    if (runs_.size() == 1) {
+      const RunMeta m = read_meta(runs_[0], s);
+      if (!m.tombs) return {runs_[0], m.count, false};
+    }
+    const Run merged = merge_all(runs_, /*consume=*/false, s);
+    return {merged, read_count(merged, s), true};
   }
 
   // Epoch boundary: survivors must fit the capacity (GPULSMOpt.cuh:7350).
