@@ -389,6 +389,12 @@ __global__ __launch_bounds__(kFinThreads) void finalize_batch_kernel(
 // passes, with the whole batch as one tile), newest-wins dedupe, value
 // gather, encode, and the radix directory.  Replaces nine launches for the
 // small arrivals of a serving stream.
+//
+// One workgroup on an empty chip: its time is its chain of barriers and memory
+// round trips.  So a short batch is spread over all eight waves (by itself 700
+// keys filled two, with eight items in a row each), digits that do not vary are
+// skipped, and keys, values and flags are all read before the sort.  700
+// updates: 20.7 us before, 11.7 so.
 constexpr int kSmallThreads = 512;
 constexpr int kSmallWaves = kSmallThreads / kWave;
 
@@ -427,81 +433,111 @@ __device__ __forceinline__ void small_batch_run(
   __shared__ unsigned short s_p0[kTile];
   __shared__ unsigned short s_p1[kTile];
   __shared__ u32 s_hist[kSmallWaves * 256];
-  __shared__ u32 s_start[256];
-  __shared__ u32 s_scan[32];
+  __shared__ u32 s_scan[kSmallWaves];
   __shared__ u32 s_misc[8];
+  __shared__ K s_vary;  // the bits that vary among the keys
+  constexpr u32 kSmallErased = 0x8000u;
+  static_assert(kTile <= 0x8000, "positions below the erase flag");
   const u32 tid = threadIdx.x;
   const u32 lane = lane_id();
   const u32 wave = tid / kWave;
+  // items per thread: a short batch is spread over all waves
+  const u32 ipt = __builtin_amdgcn_readfirstlane((n + kSmallThreads - 1) /
+                                                 kSmallThreads);
+  const u32 wave_base = wave * (kWave * ipt);
 
-  for (u32 i = tid; i < n; i += kSmallThreads) {
-    s_k0[i] = batch.key(i);
-    s_p0[i] = static_cast<unsigned short>(i);
-  }
-  __syncthreads();
-  K *src_k = s_k0, *dst_k = s_k1;
-  unsigned short *src_p = s_p0, *dst_p = s_p1;
-  for (int pass = 0; pass < kPasses; ++pass) {
-    const u32 shift = 8u * pass;
-    for (u32 i = tid; i < kSmallWaves * 256; i += kSmallThreads) s_hist[i] = 0;
-    __syncthreads();
+  // everything of the batch is read here, at once: keys, erase flags (in the
+  // positions' top bit) and values (item j of thread t: update j * 512 + t)
+  V value[kItems];
+  {
     K key[kItems];
-    u32 pos[kItems], rank[kItems];
-    u32 *my_hist = s_hist + wave * 256;
+    u32 erased = 0;
 #pragma unroll
     for (int j = 0; j < kItems; ++j) {
-      const u32 idx = wave * (kWave * kItems) + j * kWave + lane;
+      const u32 i = j * kSmallThreads + tid;
+      key[j] = 0;
+      value[j] = 0;
+      if (i < n) {
+        key[j] = batch.key(i);
+        // (an erase has no value to read)
+        if (mode == kModeErase || (mode == kModeMixed && batch.erased(i)))
+          erased |= 1u << j;
+        else
+          value[j] = batch.value(i);
+      }
+    }
+    if (tid == 0) {
+      s_k0[0] = key[0];
+      s_vary = 0;
+    }
+    __syncthreads();
+    const K first = s_k0[0];
+    K vary = 0;
+#pragma unroll
+    for (int j = 0; j < kItems; ++j) {
+      const u32 i = j * kSmallThreads + tid;
+      if (i < n) {
+        vary |= key[j] ^ first;
+        if (i) s_k0[i] = key[j];
+        s_p0[i] = static_cast<unsigned short>(
+            i | ((erased >> j) & 1u ? kSmallErased : 0u));
+      }
+    }
+#pragma unroll
+    for (int o = kWave / 2; o > 0; o >>= 1) vary |= __shfl_xor(vary, o, kWave);
+    if (lane == 0 && vary) atomicOr(&s_vary, vary);
+    __syncthreads();
+  }
+  const K vary = s_vary;
+  K *src_k = s_k0, *dst_k = s_k1;
+  unsigned short *src_p = s_p0, *dst_p = s_p1;
+  u32 *my_hist = s_hist + wave * 256;
+  for (int pass = 0; pass < kPasses; ++pass) {
+    const u32 shift = 8u * pass;
+    if (((vary >> shift) & K(0xff)) == 0) continue;  // (uniform)
+    for (u32 i = lane; i < 256; i += kWave) lds_store(&my_hist[i], 0);
+    __builtin_amdgcn_wave_barrier();
+    K key[kItems];
+    u32 pos[kItems], rank[kItems];
+#pragma unroll
+    for (int j = 0; j < kItems; ++j) {
+      if (static_cast<u32>(j) >= ipt) continue;
+      const u32 idx = wave_base + j * kWave + lane;
       const bool valid = idx < n;
       key[j] = valid ? src_k[idx] : T::kAllOnes;
       pos[j] = valid ? src_p[idx] : 0u;
       const u32 d = static_cast<u32>(key[j] >> shift) & 0xffu;
-      u64 match = ballot(valid);
-#pragma unroll
-      for (int b = 0; b < 8; ++b) {
-        const bool bit = (d >> b) & 1u;
-        const u64 vote = ballot(bit);
-        match &= bit ? vote : ~vote;
-      }
-      u32 prior = 0;
-      if (valid) prior = lds_load(&my_hist[d]);
-      rank[j] = prior + popc64(match & lanemask_lt());
-      if (valid && (match >> lane) == 1ull)
-        lds_store(&my_hist[d], prior + popc64(match));
+      rank[j] = count_peers(&my_hist[d], digit_peers(d, ballot(valid)), valid);
     }
     __syncthreads();
-    // wave prefixes per digit (threads 0..255 own one digit each)
-    u32 total = 0;
+    // a digit per thread (threads 0..255): its counts in the waves, its start
+    u32 c[kSmallWaves], total = 0;
     if (tid < 256) {
+#pragma unroll
       for (int w = 0; w < kSmallWaves; ++w) {
-        const u32 c = s_hist[w * 256 + tid];
-        s_hist[w * 256 + tid] = total;
-        total += c;
+        c[w] = s_hist[w * 256 + tid];
+        total += c[w];
       }
     }
-    // exclusive scan of the digit totals over 256 digits
-    {
-      const u32 v = tid < 256 ? total : 0u;
-      const u32 inc = wave_inclusive_scan(v);
-      if (lane == kWave - 1) s_scan[wave] = inc;
-      __syncthreads();
-      if (tid == 0) {
-        u32 run = 0;
-        for (int w = 0; w < kSmallWaves; ++w) {
-          const u32 t = s_scan[w];
-          s_scan[w] = run;
-          run += t;
-        }
+    const u32 inclusive = wave_inclusive_scan(total);
+    if (tid < 256 && lane == kWave - 1) s_scan[wave] = inclusive;
+    __syncthreads();
+    if (tid < 256) {
+      u32 start = inclusive - total;
+      for (u32 w = 0; w < wave; ++w) start += s_scan[w];
+#pragma unroll
+      for (int w = 0; w < kSmallWaves; ++w) {
+        s_hist[w * 256 + tid] = start;
+        start += c[w];
       }
-      __syncthreads();
-      if (tid < 256) s_start[tid] = s_scan[wave] + inc - v;
     }
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < kItems; ++j) {
-      const u32 idx = wave * (kWave * kItems) + j * kWave + lane;
-      if (idx < n) {
+      if (static_cast<u32>(j) >= ipt) continue;
+      if (wave_base + j * kWave + lane < n) {
         const u32 d = static_cast<u32>(key[j] >> shift) & 0xffu;
-        const u32 lp = s_start[d] + s_hist[wave * 256 + d] + rank[j];
+        const u32 lp = my_hist[d] + rank[j];
         dst_k[lp] = key[j];
         dst_p[lp] = static_cast<unsigned short>(pos[j]);
       }
@@ -515,8 +551,12 @@ __device__ __forceinline__ void small_batch_run(
     dst_p = tp;
   }
   // sorted (key, position) in src_*; keep the last occurrence of each key.
-  // Survivor ranks: ballots per (item row j, wave), scanned by thread 0.
+  // Survivor ranks: ballots per (item row j, wave), scanned by wave 0.  The
+  // values go to the array that the sort has left, by position.
   u32 *s_off = s_hist;  // reuse: kItems * kSmallWaves words
+  static_assert(kItems * kSmallWaves <= kWave, "scanned by a wave");
+  static_assert(sizeof(V) == sizeof(K), "values in the keys' array");
+  V *s_val = reinterpret_cast<V *>(dst_k);
   u64 mask[kItems];
 #pragma unroll
   for (int j = 0; j < kItems; ++j) {
@@ -524,41 +564,46 @@ __device__ __forceinline__ void small_batch_run(
     const bool keep = i < n && (i + 1 == n || src_k[i + 1] != src_k[i]);
     mask[j] = ballot(keep);
     if (lane == 0) s_off[j * kSmallWaves + wave] = popc64(mask[j]);
+    if (i < n) s_val[i] = value[j];
   }
   __syncthreads();
-  if (tid == 0) {
-    u32 run = 0;
-    for (int k = 0; k < kItems * kSmallWaves; ++k) {
-      const u32 c = s_off[k];
-      s_off[k] = run;
-      run += c;
+  if (wave == 0) {
+    const u32 v = lane < kItems * kSmallWaves ? s_off[lane] : 0u;
+    const u32 inc = wave_inclusive_scan(v);
+    if (lane < kItems * kSmallWaves) s_off[lane] = inc - v;
+    if (lane == kWave - 1) s_misc[0] = inc;  // count
+    if (lane == 0) {
+      s_misc[1] = 0;  // split
+      s_misc[2] = 0;  // tombs
     }
-    s_misc[0] = run;  // count
-    s_misc[1] = 0;    // split
-    s_misc[2] = 0;    // tombs
   }
   __syncthreads();
   const u32 count = s_misc[0];
   u32 low = 0, tombs = 0;
-  // decoded output keys go to dst_k for the directory pass
+  K kept[kItems];
+  u32 at[kItems];
 #pragma unroll
   for (int j = 0; j < kItems; ++j) {
+    at[j] = ~0u;
     if (!((mask[j] >> lane) & 1ull)) continue;
     const u32 i = j * kSmallThreads + tid;
     const u32 o = s_off[j * kSmallWaves + wave] +
                   popc64(mask[j] & lanemask_lt());
     const K k = src_k[i];
     const u32 p = src_p[i];
-    bool tomb;
-    if (mode == kModeErase) tomb = true;
-    else if (mode == kModeMixed) tomb = batch.erased(p);
-    else tomb = false;
+    const bool tomb = (p & kSmallErased) != 0;
     out[o] = T::make((k & T::kLow) | (tomb ? T::kTomb : K(0)),
-                     tomb ? V(0) : batch.value(p));
-    dst_k[o] = k;
+                     tomb ? V(0) : s_val[p & (kSmallErased - 1)]);
+    kept[j] = k;
+    at[j] = o;
     low += k < T::kTomb;
     tombs += tomb;
   }
+  __syncthreads();  // the values are read
+  // decoded output keys go to dst_k for the directory pass
+#pragma unroll
+  for (int j = 0; j < kItems; ++j)
+    if (at[j] != ~0u) dst_k[at[j]] = kept[j];
   low = wave_sum_u32(low);
   tombs = wave_sum_u32(tombs);
   if (lane == 0) {
