@@ -96,10 +96,9 @@ class FlixImpl : public FlixBase {
       Lease<V> uv(pool_, std::max<u64>(n, 1));
       u64 m = 0;
       if (n) {
-        Lease<u64> offs;
-        sort_unique(keys, nullptr, n, /*positions=*/true, nullptr, uk.get(),
-                    uv.get(), offs, s);
-        GD_HIP(hipMemcpyAsync(&m, offs.get() + n, sizeof(u64),
+        Lease<u64> unique;
+        sort_unique(keys, nullptr, n, nullptr, uk.get(), uv.get(), unique, s);
+        GD_HIP(hipMemcpyAsync(&m, unique.get(), sizeof(u64),
                               hipMemcpyDeviceToHost, s));
         GD_HIP(hipStreamSynchronize(s));
       }
@@ -133,12 +132,11 @@ class FlixImpl : public FlixBase {
       Lease<K> bk(pool_, n);
       Lease<V> bv(pool_, n);
       const Pool<K, V> existing = pool_view();
-      // the new keys' count stays on the device (offs[n]): the plan reads
+      // the new keys' count stays on the device: the plan reads
       // it there, and the plan's own read-back is the call's only wait
-      Lease<u64> offs;
-      sort_unique(keys, vals, n, false, &existing, bk.get(), bv.get(), offs,
-                  s);
-      apply_insert(bk.get(), bv.get(), offs.get() + n, n, s);
+      Lease<u64> fresh;
+      sort_unique(keys, vals, n, &existing, bk.get(), bv.get(), fresh, s);
+      apply_insert(bk.get(), bv.get(), fresh.get(), n, s);
     } catch (...) {
       order_.end(s);
       throw;
@@ -404,34 +402,35 @@ class FlixImpl : public FlixBase {
 
   // Sorts (key, position), keeps the first occurrence of each key (and, when
   // `existing` is given, only keys not yet stored), compacts into (ok, ov)
-  // with values gathered from `vals` (or = input positions).  offs receives
-  // n + 1 words, the rows' positions; offs[n] = the number of rows (on the
-  // device: nothing here waits for it).
-  void sort_unique(const K *keys, const V *vals, u64 n, bool positions,
-                   const Pool<K, V> *existing, K *ok, V *ov, Lease<u64> &offs,
+  // with values gathered from `vals` (null: the input positions).  count
+  // receives a word, the number of rows (on the device: nothing here waits
+  // for it).
+  void sort_unique(const K *keys, const V *vals, u64 n,
+                   const Pool<K, V> *existing, K *ok, V *ov, Lease<u64> &count,
                    hipStream_t s) {
     const u32 nn = static_cast<u32>(n);
     Lease<K> ka(pool_, n), kb(pool_, n);
     Lease<u32> va(pool_, n), vb(pool_, n);
-    Lease<u32> ctrl(pool_, rs::control_words(n, rs::passes_for<K>()));
+    // [sort | ticket, pad | a status word per tile], cleared together
+    const u32 tiles =
+        static_cast<u32>((n + kUniqueTile - 1) / kUniqueTile);
+    const u64 sort_words = rs::control_words(n, rs::passes_for<K>());
+    const u64 words = sort_words + 64 + 2ull * tiles;
+    Lease<u32> ctrl(pool_, words);
+    u32 *ticket = ctrl.get() + sort_words;
     GD_HIP(rs::sort_pairs<K>(keys, nn, ka.get(), va.get(), kb.get(), vb.get(),
-                             ctrl.get(), s));
-    Lease<u32> keep(pool_, n);
+                             ctrl.get(), s, 0, words));
+    Lease<u32> keep;
     if (existing) {
+      keep = Lease<u32>(pool_, n);
       mark_new_kernel<K, V><<<grid_for(n, 256, 1u << 16), 256, 0, s>>>(
           *existing, ka.get(), n, keep.get());
-    } else {
-      mark_first_kernel<K><<<grid_for(n, 256, 1u << 16), 256, 0, s>>>(
-          ka.get(), n, keep.get());
+      GD_LAUNCH_CHECK();
     }
-    GD_LAUNCH_CHECK();
-    Lease<u64> keep64(pool_, n + 1);
-    widen(keep.get(), n, keep64.get(), s);
-    offs = Lease<u64>(pool_, n + 1);
-    exclusive_scan(keep64.get(), n, offs.get(), s);
-    compact_batch_kernel<K, V><<<grid_for(n, 256, 1u << 16), 256, 0, s>>>(
-        ka.get(), va.get(), n, keep.get(), offs.get(), vals,
-        positions ? 1 : 0, ok, ov);
+    count = Lease<u64>(pool_, 1);
+    unique_batch_kernel<K, V><<<tiles, kUniqueThreads, 0, s>>>(
+        ka.get(), va.get(), nn, existing ? keep.get() : nullptr, vals, ok, ov,
+        count.get(), reinterpret_cast<u64 *>(ticket + 64), ticket);
     GD_LAUNCH_CHECK();
   }
 

@@ -1225,30 +1225,84 @@ static __global__ __launch_bounds__(256) void scan_u64_kernel(const u64 *in, u64
   }
 }
 
-// Compacts the marked rows of a sorted batch and gathers their values
-// (sorted positions sp index the caller's value array; build passes values
-// = positions themselves).
+// The first occurrence of every key of a stably sorted batch (keep null), or
+// the keys that keep[] marks, in order: (ok, ov) with values gathered (values
+// null: the input positions), *total = their number.  A tile of kUniqueTile
+// keys per workgroup, in ticket order; a chained scan gives its offset.  Items
+// are striped (item j of a thread is base + j * 512 + tid).
+//
+// It streams the batch once.  Marks, their widening to 64 bits, a scan of them
+// and the compaction, a launch each, moved six times the bytes: 8,388,608
+// 32-bit keys 140 us, 55 so.
+constexpr int kUniqueThreads = 512;
+constexpr int kUniqueItems = 8;
+constexpr int kUniqueTile = kUniqueThreads * kUniqueItems;
 template <class K, class V>
-static __global__ void compact_batch_kernel(const K *sk, const u32 *sp, u64 n,
-                                     const u32 *keep, const u64 *offs,
-                                     const V *values, int values_are_positions,
-                                     K *ok, V *ov) {
-  const u64 stride = u64(gridDim.x) * blockDim.x;
-  for (u64 i = u64(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
-       i += stride) {
-    if (!keep[i]) continue;
-    const u64 o = offs[i];
-    ok[o] = sk[i];
-    ov[o] = values_are_positions ? static_cast<V>(sp[i]) : values[sp[i]];
+static __global__ __launch_bounds__(kUniqueThreads) void unique_batch_kernel(
+    const K *__restrict__ sk, const u32 *__restrict__ sp, u32 n,
+    const u32 *__restrict__ keep, const V *__restrict__ values,
+    K *__restrict__ ok, V *__restrict__ ov, u64 *total, u64 *status,
+    u32 *ticket) {
+  constexpr int kWaves = kUniqueThreads / kWave;
+  static_assert(kUniqueItems * kWaves == kWave, "scanned by a wave");
+  __shared__ u32 s_tile;
+  __shared__ u32 s_off[kUniqueItems * kWaves];
+  __shared__ u64 s_base;
+  const u32 tid = threadIdx.x, lane = lane_id(), wave = tid / kWave;
+  if (tid == 0) s_tile = atomicAdd(ticket, 1u);
+  __syncthreads();
+  const u32 tile = s_tile;
+  const u32 base = tile * kUniqueTile;  // below n
+  const u32 count =
+      n - base < u32(kUniqueTile) ? n - base : u32(kUniqueTile);
+  K key[kUniqueItems];
+  u32 pos[kUniqueItems];
+  u32 mine = 0;
+#pragma unroll
+  for (int j = 0; j < kUniqueItems; ++j) {
+    const u32 i = j * kUniqueThreads + tid;
+    key[j] = 0;
+    pos[j] = 0;
+    bool fresh = false;
+    if (i < count) {
+      key[j] = sk[base + i];
+      pos[j] = sp[base + i];
+      fresh = keep ? keep[base + i] != 0
+                   : base + i == 0 || sk[base + i - 1] != key[j];
+    }
+    const u64 m = ballot(fresh);
+    mine |= fresh ? 1u << j : 0u;
+    if (lane == 0) s_off[j * kWaves + wave] = popc64(m);
   }
-}
-
-// Keeps the first occurrence of every key of a stably sorted batch.
-template <class K>
-static __global__ void mark_first_kernel(const K *sk, u64 n, u32 *keep) {
-  const u64 stride = u64(gridDim.x) * blockDim.x;
-  for (u64 i = u64(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += stride)
-    keep[i] = (i == 0 || sk[i - 1] != sk[i]) ? 1u : 0u;
+  V val[kUniqueItems];
+#pragma unroll
+  for (int j = 0; j < kUniqueItems; ++j) {
+    val[j] = static_cast<V>(pos[j]);
+    if (values && ((mine >> j) & 1u)) val[j] = values[pos[j]];
+  }
+  __syncthreads();
+  if (wave == 0) {
+    const u32 c = s_off[lane];
+    const u32 inc = wave_inclusive_scan(c);
+    s_off[lane] = inc - c;
+    const u32 all = __shfl(inc, kWave - 1, kWave);
+    const u64 ex = wave_lookback(status, tile, all);
+    if (lane == 0) {
+      s_base = ex;
+      if (base + count == n) *total = ex + all;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < kUniqueItems; ++j) {
+    const u64 m = ballot((mine >> j) & 1u);
+    if ((mine >> j) & 1u) {
+      const u64 o = s_base + s_off[j * kWaves + wave] +
+                    popc64(m & lanemask_lt());
+      ok[o] = key[j];
+      ov[o] = val[j];
+    }
+  }
 }
 
 // Buckets with a non-empty batch slice -> compact work list of `room` entries
