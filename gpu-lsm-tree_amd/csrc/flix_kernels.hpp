@@ -63,7 +63,9 @@ struct Ring {
 template <class K, class V>
 __device__ __forceinline__ u32 bucket_of(const Pool<K, V> &p, K key) {
   const u64 j = static_cast<u64>(key) >> p.bdir_shift;
-  u32 lo = p.bdir[j], hi = p.bdir[j + 1];
+  u64 both;  // (one load)
+  __builtin_memcpy(&both, p.bdir + j, sizeof(both));
+  u32 lo = static_cast<u32>(both), hi = static_cast<u32>(both >> 32);
   while (lo < hi) {
     const u32 mid = (lo + hi) >> 1;
     if (p.maxv[mid] < key) lo = mid + 1;
@@ -132,12 +134,30 @@ __device__ __forceinline__ u64 lower_bound_g(const K *a, u64 lo, u64 hi,
   return lo;
 }
 
-// First slot of a node's c ascending keys whose key >= key, in two rounds
-// of independent loads instead of log2(c) dependent ones: the last key of
-// every 8-slot block (at most 8 of them, S <= 64) picks the block, then the
-// block's keys give the slot.
+// The 8-slot block from slot `base` on of a node of S slots and c keys: k[j] is
+// its slot's key where base + j < c, else anything.  A thread per query is bound
+// by its load instructions (64 addresses each), so where the slots allow it the
+// block is read 16 bytes at a time.
 template <class K>
-__device__ __forceinline__ u32 node_lower_bound(const K *nk, u32 c, K key) {
+__device__ __forceinline__ void node_block(const K *nk, u32 base, u32 c, u32 S,
+                                           K (&k)[8]) {
+  if (S % 8 == 0) {  // whole blocks, aligned; the first one when base = c = S
+    const uint4 *at = reinterpret_cast<const uint4 *>(nk + (base < c ? base : 0));
+    uint4 w[sizeof(K) / 2];
+#pragma unroll
+    for (u32 j = 0; j < sizeof(K) / 2; ++j) w[j] = at[j];
+    __builtin_memcpy(k, w, sizeof(w));
+  } else {
+#pragma unroll
+    for (u32 j = 0; j < 8; ++j) k[j] = base + j < c ? nk[base + j] : K(0);
+  }
+}
+
+// The block of a node that holds the first of its c ascending keys at or above
+// key, in one round of independent loads: the last key of every full block (at
+// most 8 of them, S <= 64).
+template <class K>
+__device__ __forceinline__ u32 node_block_of(const K *nk, u32 c, K key) {
   u32 blk = 0;
   if (c > 8) {
     K last[8];
@@ -149,45 +169,61 @@ __device__ __forceinline__ u32 node_lower_bound(const K *nk, u32 c, K key) {
 #pragma unroll
     for (u32 j = 0; j < 8; ++j) blk += (8 * j + 7 < c && last[j] < key);
   }
-  const u32 base = 8 * blk;
-  K k[8];
-#pragma unroll
-  for (u32 j = 0; j < 8; ++j) k[j] = base + j < c ? nk[base + j] : K(0);
-  u32 below = 0;
-#pragma unroll
-  for (u32 j = 0; j < 8; ++j) below += (base + j < c && k[j] < key);
-  return base + below;
+  return blk;
 }
 
-// node_lower_bound with fewer loads and more rounds: a binary search over
-// the last keys of the node's full 8-slot blocks (one load per round, at
-// most four rounds), then the chosen block's keys.  Queries in random order
-// miss the caches, and a thread per query is bound by its loads more than
-// by its rounds there; queries in key order find the node's lines in cache
-// and take node_lower_bound's single round of block lasts.
+// The same with fewer loads and more rounds: a binary search over the full
+// blocks' last keys (one load per round, at most four rounds).  Queries in
+// random order miss the caches, and a thread per query is bound by its loads
+// more than by its rounds there; queries in key order find the node's lines in
+// cache and take node_block_of's single round.
 template <class K>
-__device__ __forceinline__ u32 node_lower_bound_bisect(const K *nk, u32 c,
-                                                       K key) {
+__device__ __forceinline__ u32 node_block_bisect(const K *nk, u32 c, K key) {
   u32 blk = 0, hi = c >> 3;
   while (blk < hi) {
     const u32 mid = (blk + hi) >> 1;
     if (nk[8 * mid + 7] < key) blk = mid + 1;
     else hi = mid;
   }
-  const u32 base = 8 * blk;
+  return blk;
+}
+
+// First slot of a node's c ascending keys whose key >= key, in two rounds of
+// loads instead of log2(c) dependent ones.
+template <class K>
+__device__ __forceinline__ u32 node_lower_bound(const K *nk, u32 c, u32 S,
+                                                K key) {
+  const u32 base = 8 * node_block_of(nk, c, key);
   K k[8];
-#pragma unroll
-  for (u32 j = 0; j < 8; ++j) k[j] = base + j < c ? nk[base + j] : K(0);
+  node_block(nk, base, c, S, k);
   u32 below = 0;
 #pragma unroll
   for (u32 j = 0; j < 8; ++j) below += (base + j < c && k[j] < key);
   return base + below;
 }
 
+// Whether a node holds key, and in which slot.
+template <class K>
+__device__ __forceinline__ bool node_find(const K *nk, u32 base, u32 c, u32 S,
+                                          K key, u32 &slot) {
+  K k[8];
+  node_block(nk, base, c, S, k);
+  bool hit = false;
+#pragma unroll
+  for (u32 j = 0; j < 8; ++j) {
+    if (base + j < c && k[j] == key) {
+      hit = true;
+      slot = base + j;
+    }
+  }
+  return hit;
+}
+
 // Slots of a node's c ascending keys that hold a key <= key (the first slot
 // above it), by the same two rounds as node_lower_bound.
 template <class K>
-__device__ __forceinline__ u32 node_upper_bound(const K *nk, u32 c, K key) {
+__device__ __forceinline__ u32 node_upper_bound(const K *nk, u32 c, u32 S,
+                                                K key) {
   u32 blk = 0;
   if (c > 8) {
     K last[8];
@@ -201,8 +237,7 @@ __device__ __forceinline__ u32 node_upper_bound(const K *nk, u32 c, K key) {
   }
   const u32 base = 8 * blk;
   K k[8];
-#pragma unroll
-  for (u32 j = 0; j < 8; ++j) k[j] = base + j < c ? nk[base + j] : K(0);
+  node_block(nk, base, c, S, k);
   u32 upto = 0;
 #pragma unroll
   for (u32 j = 0; j < 8; ++j) upto += (base + j < c && k[j] <= key);
@@ -354,8 +389,8 @@ static __global__ void mark_new_kernel(Pool<K, V> p, const K *batch, u64 n,
       const u32 node = owner_node(p, b, key);
       const u32 c = p.count[node];
       const K *nk = p.keys + u64(node) * p.S;
-      const u32 lo = node_lower_bound(nk, c, key);
-      if (lo < c && nk[lo] == key) fresh = false;
+      u32 slot = 0;
+      fresh = !node_find(nk, 8 * node_block_of(nk, c, key), c, p.S, key, slot);
     }
     keep[i] = fresh ? 1u : 0u;
   }
@@ -899,9 +934,10 @@ static __global__ void lookup_kernel(Pool<K, V> p, const K *q, u64 n, V *out) {
     const u32 node = owner_node(p, b, key);
     const u32 c = p.count[node];
     const K *nk = p.keys + u64(node) * p.S;
-    const u32 lo = node_lower_bound(nk, c, key);
-    out[i] = (lo < c && nk[lo] == key) ? p.vals[u64(node) * p.S + lo]
-                                       : ~V(0);
+    u32 slot = 0;
+    out[i] = node_find(nk, 8 * node_block_of(nk, c, key), c, p.S, key, slot)
+                 ? p.vals[u64(node) * p.S + slot]
+                 : ~V(0);
   }
 }
 
@@ -924,9 +960,10 @@ static __global__ void lookup_grouped_kernel(Pool<K, V> p, const K *qk, u64 n,
     const u32 node = owner_node(p, b, key);
     const u32 c = p.count[node];
     const K *nk = p.keys + u64(node) * p.S;
-    const u32 lo = node_lower_bound_bisect(nk, c, key);
-    res[i] = (lo < c && nk[lo] == key) ? p.vals[u64(node) * p.S + lo]
-                                       : ~V(0);
+    u32 slot = 0;
+    res[i] = node_find(nk, 8 * node_block_bisect(nk, c, key), c, p.S, key, slot)
+                 ? p.vals[u64(node) * p.S + slot]
+                 : ~V(0);
   }
 }
 
@@ -1008,7 +1045,7 @@ __device__ __forceinline__ void ceiling_position(const Pool<K, V> &p, K key,
   while (true) {
     const u32 c = p.count[node];
     const K *nk = p.keys + u64(node) * p.S;
-    const u32 lo = node_lower_bound(nk, c, key);
+    const u32 lo = node_lower_bound(nk, c, p.S, key);
     if (lo < c) {
       node_out = node;
       slot_out = lo;
@@ -1063,8 +1100,8 @@ __device__ __forceinline__ u64 rank_of(const Pool<K, V> &p, const u64 *bprefix,
   }
   const u32 c = p.count[node];
   const K *nk = p.keys + u64(node) * p.S;
-  return r + (kInclusive ? node_upper_bound(nk, c, key)
-                         : node_lower_bound(nk, c, key));
+  return r + (kInclusive ? node_upper_bound(nk, c, p.S, key)
+                         : node_lower_bound(nk, c, p.S, key));
 }
 
 // Count pass of the range enumeration: |[lo, hi]| = rank(<= hi) - rank(< lo),
