@@ -1363,19 +1363,14 @@ __host__ __device__ __forceinline__ u32 range_queries_per_wave(u32 runs) {
 // Queries per wave round of a launch of n queries: fewer than the lanes
 // allow while that keeps fewer than kRangeSpread waves busy (a few thousand
 // queries of a handful of runs would otherwise fill a fraction of the chip;
-// with twice as many waves, narrow queries take a second turn on it).  In a
-// dictionary of more than kRangeWideRows rows, whose queries may be long, up to
-// kRangeWideQueries queries are spread over twice as many (12,000 ranges of
-// 2^4 to 2^24 keys over 6 million rows: 2.2 ms and 1.7 so; four times as many
-// give 1.5, but 23,273 narrow ones took 40 us instead of 14).
+// with more waves, narrow queries, whose waves then resolve a few bounds each
+// on mostly idle lanes, take a second turn on it).  12,000 ranges of 2^4 to
+// 2^24 keys over 6 million rows would gain from 8192 waves (2.3 -> 1.5 ms), but
+// 8,153 narrow ones over 240,860 rows then take 20 us instead of 11.
 constexpr u64 kRangeSpread = 2048;
-constexpr u64 kRangeWideSpread = 4096;
-constexpr u64 kRangeWideRows = u64(1) << 17;
-constexpr u64 kRangeWideQueries = u64(1) << 14;
-inline u32 range_round(u64 n, u32 runs, u64 rows) {
+inline u32 range_round(u64 n, u32 runs) {
   const u64 most = range_queries_per_wave(runs);
-  const bool wide = rows > kRangeWideRows && n <= kRangeWideQueries;
-  const u64 even = n / (wide ? kRangeWideSpread : kRangeSpread);
+  const u64 even = (n + kRangeSpread / 2) / kRangeSpread;
   return static_cast<u32>(even < 1 ? 1 : (even < most ? even : most));
 }
 

@@ -348,20 +348,21 @@ class LsmT : public HandleBase {
   // Answers n ranges over the runs of `set` on stream s.  A few queries of a
   // large dictionary, any of which may be most of it, get a team of
   // workgroups each: up to kRangeTeamBlocks in all, for at most
-  // kRangeTeamQueries queries and more than kRangeWideRows rows (fewer rows
+  // kRangeTeamQueries queries and more than kRangeTeamRows rows (fewer rows
   // take one workgroup some tens of microseconds).  The teams' sums are the
   // handle's own buffer, zero between calls (a handle's calls are ordered); a
   // stream under capture gets none, as a graph would go on using it after
   // the call.
   static constexpr u32 kRangeTeamQueries = 2048;
   static constexpr u32 kRangeTeamBlocks = 512;
+  static constexpr u64 kRangeTeamRows = u64(1) << 17;
 
   template <class IO>
   void launch_ranges(const IO &io, u64 n, const RunSet<T> &set,
                      hipStream_t s) {
     u64 rows = 0;
     for (const auto &r : runs_) rows += r.rows_ub;
-    const u32 qw = range_round(n, set.count, rows);
+    const u32 qw = range_round(n, set.count);
     const u64 waves = (n + qw - 1) / qw;
     const u32 groups = grid_for(waves, kRangeWaves, 1u << 16);
     const RangeTeam team = range_team(n, groups, rows, s);
@@ -1016,7 +1017,7 @@ class LsmT : public HandleBase {
   // The team of each of the `groups` workgroups of n ranges on stream s.
   RangeTeam range_team(u64 n, u32 groups, u64 rows, hipStream_t s) {
     RangeTeam team{1, 0, nullptr, nullptr};
-    if (n > kRangeTeamQueries || rows <= kRangeWideRows ||
+    if (n > kRangeTeamQueries || rows <= kRangeTeamRows ||
         2 * groups > kRangeTeamBlocks)
       return team;
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
