@@ -1,14 +1,15 @@
-// Stable LSD radix sort of (u32 key, u32 payload) pairs for gfx950.
+// Stable LSD radix sort of (key, u32 payload) pairs for gfx950, 32- and 64-bit
+// keys.
 //
-// One global-histogram launch computes the four 8-bit digit histograms in a
-// single read of the keys; every digit pass is then ONE launch ("onesweep"):
-// a 4096-key tile is ranked in registers with wave64 ballots (a multisplit:
-// eight ballots give each lane the mask of lanes holding the same digit),
-// tiles chain their per-digit offsets through a decoupled look-back, and the
-// tile is re-ordered in LDS so the global stores leave as contiguous runs per
-// digit.  The first pass writes payload = input position, which is what the
-// callers need for "newest wins" (a stable sort keeps equal keys in input
-// order, so the last of a run of equal keys is the newest update).
+// One global-histogram launch computes the 8-bit digit histograms in a single
+// read of the keys; every digit pass is then ONE launch ("onesweep"): a tile of
+// 4096 or 8192 keys is ranked in registers (a multisplit: digit_peers gives
+// each lane the lanes holding the same digit), tiles chain their per-digit
+// offsets through a decoupled look-back, and the tile is re-ordered in LDS so
+// the global stores leave as contiguous runs per digit.  The first pass writes
+// payload = input position, which is what the callers need for "newest wins" (a
+// stable sort keeps equal keys in input order, so the last of a run of equal
+// keys is the newest update), or takes the caller's payloads.
 #pragma once
 
 #include "device_utils.hpp"
