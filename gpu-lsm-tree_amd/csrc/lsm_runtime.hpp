@@ -377,8 +377,10 @@ class LsmT : public HandleBase {
       throw Error(GD_INVALID_ARGUMENT, "invalid GPULSMOpt successor");
     order_.begin(s);
     const RunSet<T> set = run_set();
-    successor_kernel<T><<<grid_for(n, 256, 1u << 16), 256, 0, s>>>(q, n, out,
-                                                                    set);
+    u32 group_log = 0;  // a lane per run
+    while ((1u << group_log) < set.count) ++group_log;
+    successor_kernel<T><<<grid_for(n << group_log, 256, 1u << 16), 256, 0,
+                          s>>>(q, n, out, set, group_log);
     GD_LAUNCH_CHECK();
     order_.end(s);
   }
