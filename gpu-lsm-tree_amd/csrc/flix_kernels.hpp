@@ -767,7 +767,8 @@ static __global__ void plan_reset_kernel(InsertPlan *plan) {
 // share of the slice) load while this node is searched and compacted, and the
 // searches read a window of kDeleteStage slice keys in the wave's LDS (sk),
 // which moves along with the walk.  (Only a node whose share exceeds the
-// window, keys that are mostly absent, is searched in global memory.)  1.5
+// window, keys that are mostly absent or repeated, is searched in global
+// memory, and the window is filled again behind it.)  1.5
 // million deletes of 64-bit keys, half of them in 730 chains of 33 nodes: the
 // kernel 700 -> 327 us (368 with the long slices at their places in the list; a
 // window of 512 is no faster).
@@ -830,7 +831,9 @@ __device__ __forceinline__ void delete_bucket(Pool<K, V> &p, Ring &ring,
     }
     V val = V(0);
     if (lane < c) val = p.vals[u64(node) * S + lane];
-    if (pos == w0 + wn) fill(pos);  // (pos < end)
+    // (pos < end; it is behind the window's end when the last node's share
+    // reached beyond it)
+    if (pos >= w0 + wn) fill(pos);
     // delete keys below the next node's first key (none when the slice's
     // first key is not below it)
     u64 q = end;
