@@ -1904,6 +1904,12 @@ __global__ __launch_bounds__(256) void successor_kernel(
     typename T::K *__restrict__ out, RunSet<T> runs, u32 group_log) {
   using K = typename T::K;
   __shared__ RangeRuns<T> R;
+  if (runs.count == 0) {  // no row to load
+    for (u64 i = u64(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
+         i += u64(gridDim.x) * blockDim.x)
+      out[i] = T::kAllOnes;
+    return;
+  }
   R.load(runs);
   __syncthreads();
   const u32 lane = lane_id();
@@ -1919,41 +1925,36 @@ __global__ __launch_bounds__(256) void successor_kernel(
        base += u64(gridDim.x) * per) {
     const u64 q = base + (threadIdx.x >> group_log);
     bool open = q < n;  // the same for a group's lanes
-    bool has = false, dead = false;
-    u32 p = 0;
-    K k = 0;
-    auto fetch = [&]() {
-      has = p < m.count;
-      if (has) {
-        const K w = T::kw(rows[p]);
-        k = decode_key<T>(w, p, m.split);
-        dead = (w & T::kTomb) != 0;
-      }
-    };
-    if (open && mine) {
-      p = run_lower_bound(rv, m, queries[q]);
-      fetch();
-    }
+    const K query = queries[open ? q : n - 1];
+    u32 p = mine ? run_lower_bound(rv, m, query) : 0u;
     K result = T::kAllOnes;
+    // The loop exchanges values over the whole wave, so its lanes have to stay
+    // together: a lane steps by a select and every lane loads in each round (the
+    // run's first row where it did not step or has none left: few lines).  With
+    // a branch around the step the compiler made an inner loop of the lanes that
+    // stepped, whose exchanges then missed the other lanes' keys: wrong
+    // successors.
+    bool step = open && mine;
+    K w = 0;
     while (ballot(open)) {
+      const bool has = mine && p < m.count;
+      const K x = T::kw(rows[step && has ? p : 0u]);
+      w = step ? x : w;
+      const K k = decode_key<T>(w, p, m.split);
       K best = has ? k : T::kAllOnes;
       for (u32 o = 1; o < G; o <<= 1) {
-        const K x = __shfl_xor(best, o, kWave);
-        best = x < best ? x : best;
+        const K other = __shfl_xor(best, o, kWave);
+        best = other < best ? other : best;
       }
-      const u64 holders = ballot(has && k == best) & group;
-      const u64 tombs = ballot(has && dead);
+      const bool holds = has && k == best;
+      const u64 holders = ballot(holds) & group;
+      const u64 tombs = ballot(has && (w & T::kTomb) != 0);
       const u64 newest = holders & (~holders + 1);
       const bool live = holders && !(tombs & newest);
-      if (open && live) result = best;
+      result = open && live ? best : result;
       open = open && holders && !live && best != T::kAllOnes;
-      if (open && has && k == best) {
-        ++p;
-        fetch();
-      }
-      // one back edge for all lanes: without it the compiler turned the lanes
-      // that step into a loop of their own, which the others sat out
-      __builtin_amdgcn_wave_barrier();
+      step = open && holds;
+      p += step ? 1u : 0u;
     }
     if (q < n && r == 0) out[q] = result;
   }
