@@ -347,14 +347,15 @@ class LsmT : public HandleBase {
 
   // Answers n ranges over the runs of `set` on stream s.  A few queries of a
   // large dictionary, any of which may be most of it, get a team of
-  // workgroups each: up to kRangeTeamBlocks in all, for at most
-  // kRangeTeamQueries queries and more than kRangeTeamRows rows (fewer rows
+  // workgroups per group of kRangeWaves queries: up to kRangeTeamBlocks
+  // workgroups in all, so two or more for each group of at most
+  // kRangeTeamQueries queries, over more than kRangeTeamRows rows (fewer rows
   // take one workgroup some tens of microseconds).  The teams' sums are the
   // handle's own buffer, zero between calls (a handle's calls are ordered); a
   // stream under capture gets none, as a graph would go on using it after
   // the call.
-  static constexpr u32 kRangeTeamQueries = 2048;
   static constexpr u32 kRangeTeamBlocks = 512;
+  static constexpr u32 kRangeTeamQueries = kRangeTeamBlocks / 2 * kRangeWaves;
   static constexpr u64 kRangeTeamRows = u64(1) << 17;
 
   template <class IO>
@@ -1019,9 +1020,8 @@ class LsmT : public HandleBase {
   // The team of each of the `groups` workgroups of n ranges on stream s.
   RangeTeam range_team(u64 n, u32 groups, u64 rows, hipStream_t s) {
     RangeTeam team{1, 0, nullptr, nullptr};
-    if (n > kRangeTeamQueries || rows <= kRangeTeamRows ||
-        2 * groups > kRangeTeamBlocks)
-      return team;
+    // (more queries would leave no group a second workgroup)
+    if (n > kRangeTeamQueries || rows <= kRangeTeamRows) return team;
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &capturing) != hipSuccess) {
       (void)hipGetLastError();
