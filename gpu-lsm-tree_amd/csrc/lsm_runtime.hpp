@@ -391,18 +391,15 @@ class LsmT : public HandleBase {
     u64 count = 0;
     try {
       if (!runs_.empty()) {
-        Live live = live_rows(s);
+        const Live live(*this, s);
         count = live.count;
         if (count <= capacity && count) {
-          if (!out_keys || !out_vals) {
-            if (live.merged) free_run(live.run);
+          if (!out_keys || !out_vals)
             throw Error(GD_INVALID_ARGUMENT, "null dump output");
-          }
           decode_run_kernel<T><<<grid_for(count, 256, 1u << 16), 256, 0, s>>>(
               live.run.rows, live.run.meta(), out_keys, out_vals);
           GD_LAUNCH_CHECK();
         }
-        if (live.merged) free_run(live.run);
         GD_HIP(hipStreamSynchronize(s));
       }
     } catch (...) {
@@ -445,13 +442,9 @@ class LsmT : public HandleBase {
     if (!path) throw Error(GD_INVALID_ARGUMENT, "null snapshot path");
     order_.begin(s);
     u64 count = 0;
-    // a merged copy goes back to the pool on every exit path
-    Live live{};
     try {
-      if (!runs_.empty()) {
-        live = live_rows(s);
-        count = live.count;
-      }
+      const Live live(*this, s);
+      count = live.count;
       Lease<K> k(pool_, std::max<u64>(count, 1));
       Lease<V> v(pool_, std::max<u64>(count, 1));
       if (count) {
@@ -477,10 +470,7 @@ class LsmT : public HandleBase {
       write_all(f.p, &h, sizeof(h));
       // a failed final flush (a full disk) must not report success
       f.close_checked();
-      if (live.merged) free_run(live.run);
-      live.merged = false;
     } catch (...) {
-      if (live.merged) free_run(live.run);
       order_.end(s);
       throw;
     }
@@ -1426,20 +1416,42 @@ class LsmT : public HandleBase {
 
   // The live rows as one run: the only run where it holds no tombstones (as a
   // bulk build leaves it: merging it with an empty run took 89 of a 15,000,001
-  // row dump's 130 us), else a merged copy, which the caller frees.
-  struct Live {
-    Run run;
-    u64 count;
-    bool merged;
-  };
-  Live live_rows(hipStream_t s) {
-    if (runs_.size() == 1) {
-      const RunMeta m = read_meta(runs_[0], s);
-      if (!m.tombs) return {runs_[0], m.count, false};
+  // row dump's 130 us), else a merged copy, which goes back to the pool with
+  // this object (on every exit path, a failed read-back among them).
+  class Live {
+   public:
+    Live(LsmT &lsm, hipStream_t s) : lsm_(lsm) {
+      if (lsm.runs_.empty()) return;
+      if (lsm.runs_.size() == 1) {
+        const RunMeta m = lsm.read_meta(lsm.runs_[0], s);
+        if (!m.tombs) {
+          run = lsm.runs_[0];
+          count = m.count;
+          return;
+        }
+      }
+      run = lsm.merge_all(lsm.runs_, /*consume=*/false, s);
+      merged_ = true;
+      try {
+        count = lsm.read_count(run, s);
+      } catch (...) {
+        lsm.free_run(run);
+        throw;
+      }
     }
-    const Run merged = merge_all(runs_, /*consume=*/false, s);
-    return {merged, read_count(merged, s), true};
-  }
+    ~Live() {
+      if (merged_) lsm_.free_run(run);
+    }
+    Live(const Live &) = delete;
+    Live &operator=(const Live &) = delete;
+
+    Run run{};
+    u64 count = 0;
+
+   private:
+    LsmT &lsm_;
+    bool merged_ = false;
+  };
 
   // Epoch boundary: survivors must fit the capacity (GPULSMOpt.cuh:7350).
   void epoch_capacity_check(hipStream_t s) {
