@@ -226,7 +226,7 @@ class FlixImpl : public FlixBase {
         digit_hist_kernel<K><<<rs::hist_blocks_for(n), rs::kThreads, 0, s>>>(
             qk, nn, shift_lo, lc.rows);
         rs::scan_kernel<<<1, rs::kRadix, 0, s>>>(lc.rows, 1, lc.offsets);
-        rs::launch_pass<K>(rs::chained_shape(n), qk,
+        rs::launch_pass<K>(rs::chained_shape<K, u32>(n), qk,
                            rs::PayloadPos{}, qa.get(), nullptr, nn, 0,
                            lc.offsets, lc.status, lc.tickets, s,
                            dest_lo.get(), shift_lo, nullptr);

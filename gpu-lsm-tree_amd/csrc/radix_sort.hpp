@@ -378,10 +378,13 @@ inline PassShape prefix_shape(u64 n, int block = 0) {
 // Passes whose tiles chain their offsets: the chain costs some 15 ns a tile,
 // half of a pass's time, so the tiles are 8192 keys where they still fill the
 // chip (8,388,608 32-bit keys: 73 us with tiles of 4096, 61 so; 1,500,003
-// 64-bit keys: 27 and 21; 300,000: 13.7 and 15.5).
+// 64-bit keys: 27 and 21; 300,000: 13.7 and 15.5) and where the LDS takes them.
+template <class K, class V>
+constexpr bool kWideTiles = sizeof(K) + sizeof(V) <= 12;
+template <class K, class V>
 inline PassShape chained_shape(u64 n, int block = 0) {
   if (block) return {block, 4096 / block, tiles_for(n)};
-  if (n < 600000) return {1024, 4, tiles_for(n)};
+  if (n < 600000 || !kWideTiles<K, V>) return {1024, 4, tiles_for(n)};
   return {1024, 8, static_cast<u32>((n + 8191) / 8192)};
 }
 
@@ -425,19 +428,23 @@ template <bool kGated, class K, class V, class Source>
 inline void launch_shaped_pass(const PassShape &h, const Source &src, K *dst_k,
                                V *dst_v, u32 n, const PassPlan &plan,
                                hipStream_t stream) {
-  if (h.block == 1024 && h.items == 8) {
-    if constexpr (sizeof(K) + sizeof(V) <= 12)  // (within the LDS)
+  if constexpr (kWideTiles<K, V>) {  // tiles of 8192 keys
+    if (h.block == 1024 && h.items == 8) {
       onesweep_kernel<K, V, Source, 8, 1024, kGated>
           <<<h.tiles, 1024, 0, stream>>>(src, dst_k, dst_v, n, plan);
-  } else if (h.block == 1024) {
+      return;
+    }
+  }
+  const u32 tiles = tiles_for(n);  // the others have 4096
+  if (h.block == 1024) {
     onesweep_kernel<K, V, Source, 4, 1024, kGated>
-        <<<h.tiles, 1024, 0, stream>>>(src, dst_k, dst_v, n, plan);
+        <<<tiles, 1024, 0, stream>>>(src, dst_k, dst_v, n, plan);
   } else if (h.block == 512) {
     onesweep_kernel<K, V, Source, 8, 512, kGated>
-        <<<h.tiles, 512, 0, stream>>>(src, dst_k, dst_v, n, plan);
+        <<<tiles, 512, 0, stream>>>(src, dst_k, dst_v, n, plan);
   } else {
     onesweep_kernel<K, V, Source, 16, 256, kGated>
-        <<<h.tiles, 256, 0, stream>>>(src, dst_k, dst_v, n, plan);
+        <<<tiles, 256, 0, stream>>>(src, dst_k, dst_v, n, plan);
   }
 }
 
@@ -486,7 +493,7 @@ inline hipError_t sort_pairs_cleared(const K *keys_in, u32 n, K *keys_a,
                                      int block, const Gate &gate,
                                      const u32 *vals_in = nullptr) {
   constexpr int kPasses = passes_for<K>();
-  const PassShape shape = chained_shape(n, block);
+  const PassShape shape = chained_shape<K, u32>(n, block);
   const Control c = control_layout(control, kPasses);
   histogram_kernel<K, kPasses><<<hist_blocks_for(n), kThreads, 0, stream>>>(
       keys_in, n, 0, c.rows, gate);
