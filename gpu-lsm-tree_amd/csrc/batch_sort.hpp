@@ -1,6 +1,5 @@
-// Admission of 64-bit batches (and of 32-bit ones that the segmented admission
-// does not take) in four launches instead of a radix sort's eight passes and a
-// finalize launch with a gather of the values:
+// Admission of 64-bit batches in four launches instead of a radix sort's eight
+// passes and a finalize launch with a gather of the values:
 //
 //   seg_tile_hist_kernel, seg_tile_scan_kernel (seg_admission.hpp)
 //                     the batch's top varying bit h, its keys' counts by the
@@ -17,7 +16,8 @@
 // keys that repeat thousands of times) is sorted by the radix passes instead.
 // The device decides: both sets of launches are made, and those that the
 // batch does not need return at once, so nothing waits for the host.  A batch
-// that fits the LDS whole takes batch_local_kernel alone.
+// that fits the LDS whole takes batch_local_kernel alone; so do 32-bit ones
+// (larger ones take the segmented admission).
 //
 // Batches of 700,001 uniform 64-bit updates: 190 us each by radix passes, 85 so
 // (histogram and scan 12, partition 17, local sort 26, the unused launches 30).
@@ -617,7 +617,8 @@ struct Scratch {
   u32 *pa, *pb, *control;
 };
 
-// Sorts a batch of n >= 1 updates into the run that `emit` describes.
+// Sorts a batch of n >= 1 updates (32-bit ones: at most kCap) into the run that
+// `emit` describes.
 template <class T>
 inline hipError_t admit_batch(const typename T::K *keys, u32 n,
                               const Scratch<T> &x, const LsmEmit<T> &emit,
@@ -633,37 +634,42 @@ inline hipError_t admit_batch(const typename T::K *keys, u32 n,
         input, true, n, nullptr, nullptr, nullptr, nullptr, nullptr, emit);
     return hipGetLastError();
   }
-  const Layout<K> L(n);
-  u32 *c = x.control;
-  Plan *plan = reinterpret_cast<Plan *>(c);
-  K *span = reinterpret_cast<K *>(c + L.span_at);
-  lsm::seg_tile_hist_kernel<K><<<L.tiles, rs::kThreads, 0, s>>>(
-      keys, n, c + L.hist_at, span, c, L.cleared,
-      reinterpret_cast<u32 *>(emit.meta), lsm::kMetaWords, nullptr, 0);
-  lsm::seg_tile_scan_kernel<K><<<rs::kRadix, rs::kThreads, 0, s>>>(
-      keys, n, c + L.hist_at, span, L.tiles, c + L.prefix_at, c + L.totals_at,
-      &plan->shift_top, &plan->largest);
-  V *vals = emit.mode == lsm::kModeErase ? nullptr : x.vals;
-  rs::PassPlan top{};
-  top.shift_dev = &plan->shift_top;
-  top.gate = {&plan->largest, S::kCap, false};
-  top.digit_totals = c + L.totals_at;
-  top.tile_prefix = c + L.prefix_at;
-  rs::launch_source_pass<K, V>(rs::prefix_shape<K>(n, block), input, x.ka, vals, n, top, s);
-  batch_local_kernel<S, K, V, Fn, LsmEmit<T>><<<256, S::kThreads, 0, s>>>(
-      input, false, n, x.ka, vals, plan, c + L.totals_at,
-      reinterpret_cast<u64 *>(c + L.status_at), emit);
-  // the batches that do not fit
-  const rs::Gate rest{&plan->largest, S::kCap, true};
-  const hipError_t e =
-      rs::sort_pairs_cleared<K>(keys, n, x.ka, x.pa, x.kb, x.pb,
-                                c + L.radix_at, s, block, rest);
-  if (e != hipSuccess) return e;
-  u32 *fin = c + L.finalize_at;
-  lsm::finalize_batch_kernel<T><<<L.finalize_tiles, lsm::kFinThreads, 0, s>>>(
-      x.ka, x.pa, n, emit.values, emit.flags, emit.mode, emit.out, emit.meta,
-      emit.dir, emit.dir_bits, reinterpret_cast<u64 *>(fin + 64), fin, rest);
-  return hipGetLastError();
+  if constexpr (sizeof(K) == 4) {
+    return hipErrorInvalidValue;  // (the segmented admission's)
+  } else {
+    const Layout<K> L(n);
+    u32 *c = x.control;
+    Plan *plan = reinterpret_cast<Plan *>(c);
+    K *span = reinterpret_cast<K *>(c + L.span_at);
+    lsm::seg_tile_hist_kernel<K><<<L.tiles, rs::kThreads, 0, s>>>(
+        keys, n, c + L.hist_at, span, c, L.cleared,
+        reinterpret_cast<u32 *>(emit.meta), lsm::kMetaWords, nullptr, 0);
+    lsm::seg_tile_scan_kernel<K><<<rs::kRadix, rs::kThreads, 0, s>>>(
+        keys, n, c + L.hist_at, span, L.tiles, c + L.prefix_at, c + L.totals_at,
+        &plan->shift_top, &plan->largest);
+    V *vals = emit.mode == lsm::kModeErase ? nullptr : x.vals;
+    rs::PassPlan top{};
+    top.shift_dev = &plan->shift_top;
+    top.gate = {&plan->largest, S::kCap, false};
+    top.digit_totals = c + L.totals_at;
+    top.tile_prefix = c + L.prefix_at;
+    rs::launch_source_pass<K, V>(rs::prefix_shape<K>(n, block), input, x.ka,
+                                 vals, n, top, s);
+    batch_local_kernel<S, K, V, Fn, LsmEmit<T>><<<256, S::kThreads, 0, s>>>(
+        input, false, n, x.ka, vals, plan, c + L.totals_at,
+        reinterpret_cast<u64 *>(c + L.status_at), emit);
+    // the batches that do not fit
+    const rs::Gate rest{&plan->largest, S::kCap, true};
+    const hipError_t e =
+        rs::sort_pairs_cleared<K>(keys, n, x.ka, x.pa, x.kb, x.pb,
+                                  c + L.radix_at, s, block, rest);
+    if (e != hipSuccess) return e;
+    u32 *fin = c + L.finalize_at;
+    lsm::finalize_batch_kernel<T><<<L.finalize_tiles, lsm::kFinThreads, 0, s>>>(
+        x.ka, x.pa, n, emit.values, emit.flags, emit.mode, emit.out, emit.meta,
+        emit.dir, emit.dir_bits, reinterpret_cast<u64 *>(fin + 64), fin, rest);
+    return hipGetLastError();
+  }
 }
 
 }  // namespace bs
