@@ -1391,6 +1391,20 @@ constexpr u32 kRangeLongWork = 1024;
 constexpr u32 kRangeNewerStep = 256;
 constexpr u32 kRangeOldStep = 1024;
 
+// Rows of several runs whose newest versions a wave finds in LDS, without a
+// search (range_resolve); a workgroup takes four times as many.  (A workgroup's
+// registers allow four of them per CU, and so does this LDS.)
+constexpr u32 kResolveRows = 512;
+constexpr u32 kResolveBlockRows = kRangeWaves * kResolveRows;
+
+// Runs from which on that is the faster way: a row of a newer run searches the
+// older ones one after another, two round trips each.  Sums of n ranges of w
+// rows, searching and resolving: 10 equal runs, n = 1, w = 60 23.3 and 16.9 us,
+// n = 10,000, w = 600 656 and 88; 40 runs 45 and 22, 9333 and 151; 4 runs 17.3
+// and 16.5, 266 and 106 (but n = 1, w = 3 14.7 and 15.4); 3 runs of falling size
+// n = 1025, w = 2000 47.9 and 63.0.
+constexpr u32 kResolveRuns = 4;
+
 // Workgroups that share the long queries of one group of queries: `size` of
 // them, this one being number `rank`.  Where size > 1, acc and left (one each
 // per query of the launch, zero before and after it) gather their sums.
@@ -1649,6 +1663,105 @@ __device__ __forceinline__ u64 range_chunk(const RangeRuns<T> &R,
   return acc;
 }
 
+// What the `total` rows of some queries add up to, by kLanes lanes together (a
+// wave, or the workgroup), each key's newest version alone: every row is read
+// once, into an LDS table of the queries' keys that keeps the first row of each
+// key (a query's rows come run after run, the newest first), and a row counts
+// when the table kept it.  No row waits for a search, so what is left is one
+// round of loads.
+//
+// at(f): where row f is (called for a lane's rows in ascending order): its
+// address, whether it lies behind its run's split, its query, and whether that
+// one counts.  span(q): query q's rows [begin, end).  add(q, v): called for each
+// row that counts.
+template <class T>
+struct ResolveRow {
+  const typename T::Row *row;
+  bool top, count;
+  u32 q;
+};
+template <class T, u32 kLanes, class At, class Span, class Add>
+__device__ __forceinline__ void range_resolve(typename T::K *keys, u32 *slots,
+                                              u32 total, u32 tid, At &&at,
+                                              Span &&span, Add &&add) {
+  using K = typename T::K;
+  using V = typename T::V;
+  constexpr int kItems = kResolveRows / kWave;
+  constexpr int kLoads = 4;  // rows of a lane in flight
+  auto sync = [] {
+    if constexpr (kLanes == kWave) {
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    } else {
+      __syncthreads();
+    }
+  };
+  // (else its items' LDS addresses are worked out at the kernel's start and
+  // held in registers from there)
+  asm volatile("" : "+v"(tid));
+  // at least two slots per row
+  u32 log = 7;
+  while ((1u << log) < 2 * total) ++log;
+  for (u32 i = tid; i < (1u << log); i += kLanes) slots[i] = 0;
+  V val[kItems];
+  u32 tag[kItems];  // the query, from the search on the slot (<< 8)
+#pragma unroll
+  for (int j0 = 0; j0 < kItems; j0 += kLoads) {
+    typename T::Row w[kLoads];
+    u32 top = 0, count = 0;
+#pragma unroll
+    for (int j = 0; j < kLoads; ++j) {
+      const u32 f = (j0 + j) * kLanes + tid;
+      tag[j0 + j] = 0;
+      if (f < total) {
+        const ResolveRow<T> x = at(f);
+        w[j] = *x.row;
+        top |= x.top ? 1u << j : 0u;
+        count |= x.count ? 1u << j : 0u;
+        tag[j0 + j] = x.q;
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < kLoads; ++j) {
+      const u32 f = (j0 + j) * kLanes + tid;
+      if (f < total) {
+        const K kw = T::kw(w[j]);
+        keys[f] = (kw & T::kLow) | ((top >> j) & 1u ? T::kTomb : K(0));
+        val[j0 + j] = (kw & T::kTomb) ? V(0)
+                      : (count >> j) & 1u ? V(1) : T::val(w[j]);
+      }
+    }
+  }
+  sync();
+#pragma unroll
+  for (int j = 0; j < kItems; ++j) {
+    const u32 f = j * kLanes + tid;
+    if (f < total) {
+      const uint2 own = span(tag[j]);
+      const K key = keys[f];
+      u32 x = static_cast<u32>(key);
+      if constexpr (sizeof(K) == 8) x ^= static_cast<u32>(key >> 32);
+      u32 h = (x * 0x9E3779B1u + tag[j] * 0x85EBCA77u) >> (32 - log);
+      while (true) {  // (some slot is free)
+        const u32 cur = atomicCAS(&slots[h], 0u, f + 1);
+        if (cur == 0) break;
+        if (cur > own.x && cur <= own.y && keys[cur - 1] == key) {
+          atomicMin(&slots[h], f + 1);
+          break;
+        }
+        h = (h + 1) & ((1u << log) - 1u);
+      }
+      tag[j] |= h << 8;
+    }
+  }
+  sync();
+#pragma unroll
+  for (int j = 0; j < kItems; ++j) {
+    const u32 f = j * kLanes + tid;
+    if (f < total && slots[tag[j] >> 8] == f + 1) add(tag[j] & 0xffu, val[j]);
+  }
+}
+
 // The range kernel's work on queries [q_begin, q_end) by the calling
 // workgroup, number group of a grid of groups (the range kernel's, or the
 // serving engine's step kernel taking chunks of queries), qw queries per wave
@@ -1664,6 +1777,11 @@ __device__ __forceinline__ u64 range_chunk(const RangeRuns<T> &R,
 // of a query's oldest run from its bounds when that run has no tombstones.
 // Sums are modulo 2^64 and are truncated to the value width.
 //
+// Over kResolveRuns runs or more (kResolve: compiled for them), queries with rows
+// of several runs search nothing up to kResolveBlockRows rows: a wave resolves
+// its short ones in LDS, as many at a time as fit, and the workgroup's waves one
+// of more than kResolveRows rows together (range_resolve).
+//
 // Bound by the searches, one per newer row and older run (directory entries,
 // then rows), whose lines come from beyond the L2 in a dictionary of tens of
 // megabytes, and by the rows read once.  12,000 sums (or counts) of 2^4 to
@@ -1673,7 +1791,7 @@ __device__ __forceinline__ u64 range_chunk(const RangeRuns<T> &R,
 // over one run of 2^20 rows 10 us (15).  A queue of all long queries' chunks
 // for a second launch took 0.38 ms, but its launch made every small call on a
 // large dictionary 3 to 5 us longer.
-template <class T, class IO>
+template <class T, bool kResolve, class IO>
 __device__ __forceinline__ void range_block(const IO &io, u64 q_begin,
                                             u64 q_end, const RunSet<T> &runs,
                                             u64 group, u64 groups, u32 qw,
@@ -1692,12 +1810,19 @@ __device__ __forceinline__ void range_block(const IO &io, u64 q_begin,
   __shared__ u32 s_flags[kRangeWaves][kQMax];
   __shared__ u32 s_plan[kRangeWaves][kQMax];
   __shared__ u32 s_woff[kRangeWaves][kQMax];
+  // rows resolved in LDS, their keys and table
+  __shared__ u32 s_roff[kRangeWaves][kResolve ? kQMax + 1 : 1];
   __shared__ unsigned long long s_acc[kRangeWaves][kQMax];
-  // the round's long queries (wave << 8 | query); round k counts in slot
-  // k % 3 and clears the next one, which no wave can still be reading
+  __shared__ K s_keys[kResolve ? kResolveBlockRows : 1];
+  __shared__ u32 s_slots[kResolve ? 2 * kResolveBlockRows : 1];
+  // the round's queries that all waves share (wave << 8 | query, kWhole: its
+  // rows are resolved in LDS); round k counts in slot k % 3 and clears the next
+  // one, which no wave can still be reading
+  constexpr u32 kWhole = 1u << 16;
   __shared__ u32 s_list[kRangeWaves * kQMax];
   __shared__ u32 s_long[3];
   const u32 nr = runs.count;
+  const bool resolve = kResolve && nr >= kResolveRuns;
   __syncthreads();  // a previous call's readers of R are done
   R.load(runs);
   if (threadIdx.x < 3) s_long[threadIdx.x] = 0;
@@ -1739,7 +1864,7 @@ __device__ __forceinline__ void range_block(const IO &io, u64 q_begin,
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
 
     // ---- plan of query q0 + lane (lanes below qw)
-    u32 work = 0;
+    u32 work = 0, resolved = 0;
     bool is_long = false;
     if (lane < qw) {
       const u32 flags = s_flags[wave][lane];
@@ -1760,14 +1885,27 @@ __device__ __forceinline__ void range_block(const IO &io, u64 q_begin,
             newer += bnd[2 * r + 1] - bnd[2 * r];
           u32 old_rows = bnd[2 * oldest + 1] - bnd[2 * oldest];
           plan = first | (oldest << 8);
-          if ((flags & 4u) && R.meta[oldest].tombs == 0) {
+          const u64 all = newer + old_rows;
+          const bool from_bounds = (flags & 4u) && R.meta[oldest].tombs == 0;
+          is_long = 4 * newer + (from_bounds ? 0u : old_rows) > kRangeLongWork;
+          // (rows that would search many runs one after another)
+          const bool whole =
+              resolve && newer && all > kResolveRows &&
+              all <= kResolveBlockRows &&
+              (is_long || newer * (oldest - first) > kResolveRows);
+          if (resolve && newer && all <= kResolveRows) {
+            is_long = false;
+            if (team.rank == 0) resolved = static_cast<u32>(all);
+          } else if (whole) {
+            is_long = true;
+          } else if (from_bounds) {
             base = team.rank == 0 ? old_rows : 0;
             old_rows = 0;
           }
-          is_long = 4 * newer + old_rows > kRangeLongWork;
           if (is_long)
-            s_list[atomicAdd(&s_long[turn], 1u)] = wave << 8 | lane;
-          else if (team.rank == 0)
+            s_list[atomicAdd(&s_long[turn], 1u)] =
+                wave << 8 | lane | (whole ? kWhole : 0u);
+          else if (team.rank == 0 && !resolved)
             work = static_cast<u32>(newer + old_rows);
         }
       }
@@ -1777,8 +1915,64 @@ __device__ __forceinline__ void range_block(const IO &io, u64 q_begin,
     const u32 work_inc = wave_inclusive_scan(work);
     if (lane < qw) s_woff[wave][lane] = work_inc - work;
     const u32 wend = __shfl(work_inc, kWave - 1, kWave);
+    u32 rend = 0;
+    if constexpr (kResolve) {
+      const u32 inc = wave_inclusive_scan(resolved);
+      if (lane < qw) s_roff[wave][lane + 1] = inc;
+      if (lane == 0) s_roff[wave][0] = 0;
+      rend = __shfl(inc, kWave - 1, kWave);
+    }
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+
+    // ---- the short queries whose rows are resolved in LDS, as many as fit at
+    // a time
+    if (kResolve && rend) {
+      u32 g0 = 0;
+      while (g0 < qw) {
+        const u32 *off = s_roff[wave];
+        const u32 from = __builtin_amdgcn_readfirstlane(off[g0]);
+        // the first query whose rows end behind the group's room
+        const u64 over =
+            ballot(lane < qw && off[lane + 1] - from > kResolveRows &&
+                   lane >= g0);
+        const u32 g1 = over ? static_cast<u32>(ffs64(over)) - 1 : qw;
+        const u32 total = __builtin_amdgcn_readfirstlane(off[g1]) - from;
+        if (total) {
+          u32 qi = g0, r = ~0u, first_row = 0;  // run r's rows start there
+          range_resolve<T, kWave>(
+              s_keys + wave * kResolveRows, s_slots + wave * 2 * kResolveRows,
+              total, lane,
+              [&](u32 f) -> ResolveRow<T> {
+                const u32 at = from + f;
+                while (off[qi + 1] <= at) {
+                  ++qi;
+                  r = ~0u;
+                }
+                const u32 *bnd = &s_b[wave][qi * per];
+                if (r == ~0u) {
+                  r = s_plan[wave][qi] & 0xffu;
+                  first_row = off[qi];
+                }
+                while (at - first_row >= bnd[2 * r + 1] - bnd[2 * r]) {
+                  first_row += bnd[2 * r + 1] - bnd[2 * r];
+                  ++r;
+                }
+                const u32 idx = bnd[2 * r] + (at - first_row);
+                return {R.rows(r) + idx, idx >= R.meta[r].split,
+                        (s_flags[wave][qi] & 4u) != 0, qi};
+              },
+              [&](u32 q) { return make_uint2(off[q] - from, off[q + 1] - from); },
+              [&](u32 q, typename T::V v) {
+                if (v)
+                  atomicAdd(&s_acc[wave][q], static_cast<unsigned long long>(v));
+              });
+          __builtin_amdgcn_wave_barrier();
+          __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        }
+        g0 = g1;
+      }
+    }
 
     // rows of the short queries, flattened query after query, run after run
     if (wend) {
@@ -1833,10 +2027,35 @@ __device__ __forceinline__ void range_block(const IO &io, u64 q_begin,
     const u32 longs = s_long[turn];
     if (!longs) continue;
     for (u32 l = 0; l < longs; ++l) {
-      const u32 id = s_list[l], w = id >> 8, qi = id & 0xffu;
+      const u32 id = s_list[l], w = (id >> 8) & 0xffu, qi = id & 0xffu;
       const u32 *bnd = &s_b[w][qi * per];
       const u32 first = s_plan[w][qi] & 0xffu, oldest = s_plan[w][qi] >> 8;
       const bool count = (s_flags[w][qi] & 4u) != 0;
+      if (kResolve && (id & kWhole)) {
+        if (team.rank) continue;
+        u32 total = 0;
+        for (u32 r = first; r <= oldest; ++r)
+          total += bnd[2 * r + 1] - bnd[2 * r];
+        u32 r = first, first_row = 0;
+        u64 acc = 0;
+        range_resolve<T, kRangeThreads>(
+            s_keys, s_slots, total, threadIdx.x,
+            [&](u32 f) -> ResolveRow<T> {
+              while (f - first_row >= bnd[2 * r + 1] - bnd[2 * r]) {
+                first_row += bnd[2 * r + 1] - bnd[2 * r];
+                ++r;
+              }
+              const u32 idx = bnd[2 * r] + (f - first_row);
+              return {R.rows(r) + idx, idx >= R.meta[r].split, count, 0u};
+            },
+            [&](u32) { return make_uint2(0u, total); },
+            [&](u32, typename T::V v) { acc += v; });
+        acc = wave_sum_u64(acc);
+        if (lane == 0 && acc)
+          atomicAdd(&s_acc[w][qi], static_cast<unsigned long long>(acc));
+        __syncthreads();  // the table is used again
+        continue;
+      }
       u64 newer = 0;
       for (u32 r = first; r < oldest; ++r) newer += bnd[2 * r + 1] - bnd[2 * r];
       const u64 old_rows = count && R.meta[oldest].tombs == 0
@@ -1854,10 +2073,10 @@ __device__ __forceinline__ void range_block(const IO &io, u64 q_begin,
     }
     __syncthreads();
     if (threadIdx.x < longs) {
-      const u32 id = s_list[threadIdx.x], w = id >> 8, qi = id & 0xffu;
+      const u32 id = s_list[threadIdx.x], w = (id >> 8) & 0xffu, qi = id & 0xffu;
       u64 sum = s_acc[w][qi];
-      bool last = true;
-      if (team.size > 1) {
+      bool last = !(id & kWhole) || team.rank == 0;
+      if (team.size > 1 && !(id & kWhole)) {
         // The sum must have taken this workgroup's share before `left`
         // counts it.  The value that the addition returns is waited for
         // instead of a fence, which would write back and empty the L2.
@@ -1878,14 +2097,14 @@ __device__ __forceinline__ void range_block(const IO &io, u64 q_begin,
 }
 
 // Teams of team.size consecutive workgroups (team.rank is set here).
-template <class T, class IO>
+template <class T, bool kResolve, class IO>
 __global__ __launch_bounds__(kRangeThreads) void range_kernel(
     IO io_arg, u64 n, RunSet<T> runs, u32 qw, RangeTeam team) {
   __shared__ __align__(16) char s_io[IO::kStageBytes ? IO::kStageBytes : 16];
   const IO io = io_arg.stage(s_io);  // range_block's first barrier orders it
   team.rank = blockIdx.x % team.size;
-  range_block<T, IO>(io, 0, n, runs, blockIdx.x / team.size,
-                     gridDim.x / team.size, qw, team);
+  range_block<T, kResolve>(io, 0, n, runs, blockIdx.x / team.size,
+                           gridDim.x / team.size, qw, team);
 }
 
 // Smallest live key >= query, all-ones when there is none.

@@ -367,8 +367,12 @@ class LsmT : public HandleBase {
     const u64 waves = (n + qw - 1) / qw;
     const u32 groups = grid_for(waves, kRangeWaves, 1u << 16);
     const RangeTeam team = range_team(n, groups, rows, s);
-    range_kernel<T, IO><<<groups * team.size, kRangeThreads, 0, s>>>(
-        io, n, set, qw, team);
+    if (set.count >= kResolveRuns)
+      range_kernel<T, true><<<groups * team.size, kRangeThreads, 0, s>>>(
+          io, n, set, qw, team);
+    else
+      range_kernel<T, false><<<groups * team.size, kRangeThreads, 0, s>>>(
+          io, n, set, qw, team);
     GD_LAUNCH_CHECK();
   }
 

@@ -330,7 +330,7 @@ __global__ __launch_bounds__(lsm::kRangeThreads) void step_query_kernel(
       }
     } else {
       const u64 r0 = u64(item - lc) * kStepRangeChunk;
-      lsm::range_block<T, PieceRange<T>>(
+      lsm::range_block<T, true>(
           rio, r0, std::min<u64>(n_rng, r0 + kStepRangeChunk), runs, 0, 1,
           lsm::range_queries_per_wave(runs.count),
           lsm::RangeTeam{1, 0, nullptr, nullptr});
