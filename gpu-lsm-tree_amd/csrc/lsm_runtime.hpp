@@ -88,6 +88,7 @@ class LsmT : public HandleBase {
     }
     clear_profile();
     if (prof_meta_) (void)hipHostFree(prof_meta_);
+    if (choice_) (void)hipHostFree(choice_);
     for (auto &kv : pending_) (void)hipEventDestroy(kv.second.done);
     pending_.clear();
     defer_ = false;
@@ -1086,10 +1087,13 @@ class LsmT : public HandleBase {
   // workgroup's LDS does not take whole go by segments: 12,000 uniform, hot and
   // Zipf keys 44, 52 and 72 us, by radix passes 74, 72 and 81, partitioned as
   // 64-bit batches are 73, 78 and 96.  32-bit builds above
-  // kSegmentedMax take the radix passes: their segments do not fit the LDS (a
-  // workgroup would sort each in memory).  2,500,000 uniform keys: 298 us by
-  // segments, 197 by passes; 15,000,001: 919 and 631.  (Keys that come twice
-  // each, whose segments are deduplicated first: 4,000,000 220 and 240.)
+  // kSegmentedMax take the radix passes, as their segments do not fit the LDS (a
+  // workgroup would sort each in memory), unless a sample says that they do once
+  // each has kept one update per key (build_scan_kernel).  Builds (the whole
+  // call) by segments, by passes, and as decided: 2,500,000 uniform keys 304, 205
+  // and 198 us, every key eight times 113, 200 and 141, Zipf keys 16,300, 230 and
+  // 227; 8,000,001 uniform keys 542, 376 and 374, every key eight times 220, 364
+  // and 258.
   static constexpr u32 kSegmentedMax = u32(1) << 21;
   Run sorted_run(const K *keys, const V *values, const u8 *flags, u32 n,
                  int mode, hipStream_t s) {
@@ -1116,7 +1120,9 @@ class LsmT : public HandleBase {
     const u64 fin_words = 64 + 2ull * fin_tiles;  // ticket pad + status u64
     Lease<K> ka(pool_, n), kb(pool_, n);
     Lease<u32> va(pool_, n), vb(pool_, n);
-    Lease<u32> ctrl(pool_, sort_words + fin_words);
+    // [sort | finalize | 16-byte aligned: sample, decision (32-bit builds)]
+    const u64 sample_at = (sort_words + fin_words + 3) / 4 * 4;
+    Lease<u32> ctrl(pool_, sample_at + kSampleWords + 1);
     u32 *fin_ctrl = ctrl.get() + sort_words;
     // 32-bit values of inserts ride along; else the positions do, and values
     // and flags are gathered
@@ -1126,17 +1132,76 @@ class LsmT : public HandleBase {
     }
     // the sort's clearing launch also clears the finalize state behind its
     // own and the run header
-    GD_HIP(rs::sort_pairs<K>(keys, n, ka.get(), va.get(), kb.get(), vb.get(),
-                             ctrl.get(), s, tuning_.sort_block,
-                             sort_words + fin_words,
-                             reinterpret_cast<u32 *>(r.meta()), kMetaWords,
-                             carried));
+    volatile u32 *choice = nullptr;
+    if constexpr (sizeof(K) == 4) {
+      if (tuning_.segmented_admission == 1) choice = build_choice();
+    }
+    if (choice) {
+      if constexpr (sizeof(K) == 4) {
+        u32 *state = ctrl.get();
+        BuildSample *sample = reinterpret_cast<BuildSample *>(state + sample_at);
+        u32 *word = state + sample_at + kSampleWords;
+        const rs::Control c = rs::control_layout(state, 4);
+        constexpr u32 kUndecided = 2;
+        *choice = kUndecided;
+        rs::clear_control(state, sample_at + kSampleClear, s,
+                          reinterpret_cast<u32 *>(r.meta()), kMetaWords);
+        build_count_kernel<<<rs::hist_blocks_for(n) + kSampleBlocks,
+                             rs::kThreads, 0, s>>>(keys, n, c.rows, sample);
+        build_scan_kernel<<<5, rs::kRadix, 0, s>>>(c.rows, c.offsets, sample,
+                                                   word, choice_);
+        GD_LAUNCH_CHECK();
+        auto passes = [&](int from, int to, const rs::Gate &gate) {
+          GD_HIP(rs::sort_passes<K>(keys, n, ka.get(), va.get(), kb.get(),
+                                    vb.get(), state, s, tuning_.sort_block,
+                                    gate, nullptr, carried, from, to));
+        };
+        // The device decides; the host makes the launches of one way only, and
+        // reads the decision while the device is in the first pass (which the
+        // decision closes).
+        passes(0, 1, rs::Gate{word, 0, false});
+        while (*choice == kUndecided) {
+          const hipError_t e = hipStreamQuery(s);
+          if (e == hipErrorNotReady) continue;
+          GD_HIP(e);
+          if (*choice == kUndecided)  // (all done, and no decision)
+            throw Error(GD_HIP_ERROR, "no decision from build_scan_kernel");
+        }
+        if (*choice) {
+          // (their buffers: all work on them is on this stream)
+          ka.reset();
+          kb.reset();
+          va.reset();
+          vb.reset();
+          return segmented_run(keys, values, flags, n, mode, s, r);
+        }
+        passes(1, 4, rs::Gate{});
+      }
+    } else {
+      GD_HIP(rs::sort_pairs<K>(keys, n, ka.get(), va.get(), kb.get(), vb.get(),
+                               ctrl.get(), s, tuning_.sort_block,
+                               sort_words + fin_words,
+                               reinterpret_cast<u32 *>(r.meta()), kMetaWords,
+                               carried));
+    }
     finalize_batch_kernel<T><<<fin_tiles, kFinThreads, 0, s>>>(
         ka.get(), va.get(), n, carried ? nullptr : values, flags, mode, r.rows, r.meta(),
         r.entries(), r.max_bits, reinterpret_cast<u64 *>(fin_ctrl + 64),
         fin_ctrl, rs::Gate{});
     GD_LAUNCH_CHECK();
     return r;
+  }
+
+  // The host's word for build_scan_kernel's decision, made with the first build
+  // that asks; null when there is no memory for it.
+  volatile u32 *build_choice() {
+    if (!choice_ && hipHostMalloc(reinterpret_cast<void **>(&choice_),
+                                  sizeof(u32),
+                                  hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();
+      choice_ = nullptr;
+    }
+    return choice_;
   }
 
   // Sorts a batch into run r through batch_sort.hpp.
@@ -1549,6 +1614,7 @@ class LsmT : public HandleBase {
   // the queries, which may be another than the pool's)
   DevicePool range_pool_{&usage_};
   u32 *range_sums_ = nullptr;
+  u32 *choice_ = nullptr;  // see build_choice()
   OperationOrder order_;
   std::vector<Run> runs_;  // newest first
   u32 pending_batches_ = 0;

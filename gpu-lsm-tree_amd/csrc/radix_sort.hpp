@@ -54,19 +54,19 @@ inline u32 hist_blocks_for(u64 n) {
 }
 
 // rows[kHistRows][kPasses][kRadix] (zeroed) += counts of digits
-// first .. first + kPasses - 1, digit p = (key >> 8p) & 0xff.
+// first .. first + kPasses - 1, digit p = (key >> 8p) & 0xff, by workgroup
+// `block` of `blocks`.
 template <class K, int kPasses>
-static __global__ __launch_bounds__(kThreads) void histogram_kernel(
-    const K *__restrict__ keys, u32 n, u32 first, u32 *__restrict__ rows,
-    Gate gate) {
-  if (gate.closed()) return;
+__device__ __forceinline__ void histogram_block(const K *__restrict__ keys,
+                                                u32 n, u32 first,
+                                                u32 *__restrict__ rows,
+                                                u32 block, u32 blocks) {
   __shared__ u32 s_hist[kPasses][kRadix];
   for (int i = threadIdx.x; i < kPasses * kRadix; i += kThreads)
     (&s_hist[0][0])[i] = 0;
   __syncthreads();
   const u64 round = u64(kThreads) * kHistItems;
-  for (u64 base = u64(blockIdx.x) * round; base < n;
-       base += u64(gridDim.x) * round) {
+  for (u64 base = u64(block) * round; base < n; base += u64(blocks) * round) {
     K k[kHistItems];
 #pragma unroll
     for (int j = 0; j < kHistItems; ++j) {
@@ -85,22 +85,29 @@ static __global__ __launch_bounds__(kThreads) void histogram_kernel(
     }
   }
   __syncthreads();
-  u32 *row = rows + u64(blockIdx.x % kHistRows) * kPasses * kRadix;
+  u32 *row = rows + u64(block % kHistRows) * kPasses * kRadix;
   for (int i = threadIdx.x; i < kPasses * kRadix; i += kThreads) {
     const u32 c = (&s_hist[0][0])[i];
     if (c) atomicAdd(&row[i], c);
   }
 }
 
-// Sums the kHistRows partial rows of pass blockIdx.x and writes the
-// exclusive scan over digits -> global digit offsets.  constant[p] (nullable,
-// zero before) = 1 when all n keys share the pass's digit.
-static __global__ __launch_bounds__(kRadix) void scan_kernel(
-    const u32 *__restrict__ rows, u32 passes, u32 *__restrict__ offsets,
-    Gate gate = Gate{}, u32 *constant = nullptr, u32 n = 0) {
+template <class K, int kPasses>
+static __global__ __launch_bounds__(kThreads) void histogram_kernel(
+    const K *__restrict__ keys, u32 n, u32 first, u32 *__restrict__ rows,
+    Gate gate) {
   if (gate.closed()) return;
+  histogram_block<K, kPasses>(keys, n, first, rows, blockIdx.x, gridDim.x);
+}
+
+// Sums the kHistRows partial rows of pass p and writes the exclusive scan over
+// digits -> global digit offsets, by one workgroup.  constant[p] (nullable,
+// zero before) = 1 when all n keys share the pass's digit.
+__device__ __forceinline__ void scan_block(const u32 *__restrict__ rows,
+                                           u32 passes, u32 p,
+                                           u32 *__restrict__ offsets,
+                                           u32 *constant, u32 n) {
   __shared__ u32 scratch[kRadix / kWave + 1];
-  const u32 p = blockIdx.x;
   u32 c[kHistRows];
 #pragma unroll
   for (int r = 0; r < kHistRows; ++r)
@@ -110,6 +117,13 @@ static __global__ __launch_bounds__(kRadix) void scan_kernel(
   for (int r = 0; r < kHistRows; ++r) v += c[r];
   offsets[p * kRadix + threadIdx.x] = block_exclusive_scan<kRadix>(v, scratch);
   if (constant && v == n) constant[p] = 1;
+}
+
+static __global__ __launch_bounds__(kRadix) void scan_kernel(
+    const u32 *__restrict__ rows, u32 passes, u32 *__restrict__ offsets,
+    Gate gate = Gate{}, u32 *constant = nullptr, u32 n = 0) {
+  if (gate.closed()) return;
+  scan_block(rows, passes, blockIdx.x, offsets, constant, n);
 }
 
 // Payload policies of a digit pass: payload(idx, valid, key, shift)
@@ -485,23 +499,19 @@ inline void launch_pass(const PassShape &shape, const K *src_k,
                              dst_v, n, plan, stream);
 }
 
-// sort_pairs below, without its clearing launch and behind a gate.
+// Passes from .. to - 1 of sort_pairs below, behind its clearing and counting
+// launches.  constant: nullable, see scan_block; pairs of passes over constant
+// digits are then skipped (64-bit keys of a narrow range, and behind a gate), but
+// not the first pair, which reads the input.
 template <class K>
-inline hipError_t sort_pairs_cleared(const K *keys_in, u32 n, K *keys_a,
-                                     u32 *vals_a, K *keys_b, u32 *vals_b,
-                                     u32 *control, hipStream_t stream,
-                                     int block, const Gate &gate,
-                                     const u32 *vals_in = nullptr) {
+inline hipError_t sort_passes(const K *keys_in, u32 n, K *keys_a, u32 *vals_a,
+                              K *keys_b, u32 *vals_b, u32 *control,
+                              hipStream_t stream, int block, const Gate &gate,
+                              const u32 *constant, const u32 *vals_in,
+                              int from = 0, int to = passes_for<K>()) {
   constexpr int kPasses = passes_for<K>();
   const PassShape shape = chained_shape<K, u32>(n, block);
   const Control c = control_layout(control, kPasses);
-  histogram_kernel<K, kPasses><<<hist_blocks_for(n), kThreads, 0, stream>>>(
-      keys_in, n, 0, c.rows, gate);
-  // pairs of passes over constant digits are skipped (64-bit keys of a narrow
-  // range); the first pair, which reads the input, is not
-  u32 *constant = gate.value || kPasses > 4 ? c.tickets + 32 : nullptr;
-  scan_kernel<<<kPasses, kRadix, 0, stream>>>(c.rows, kPasses, c.offsets, gate,
-                                              constant, n);
   u32 *tickets = c.tickets;
   u64 *status = c.status;
   const u32 *offsets = c.offsets;
@@ -509,9 +519,11 @@ inline hipError_t sort_pairs_cleared(const K *keys_in, u32 n, K *keys_a,
   const u32 *src_v = vals_in;
   K *dst_k = keys_b;
   u32 *dst_v = vals_b;
-  for (int p = 0; p < kPasses; ++p) {
+  for (int p = 0; p < to; ++p) {
     u64 *pass_status = status + u64(p) * tiles_for(n) * kRadix;
-    if (p == 0 && !vals_in) {
+    if (p < from) {
+      // an earlier call's
+    } else if (p == 0 && !vals_in) {
       launch_pass<K>(shape, src_k, PayloadPos{}, dst_k, dst_v, n, 0,
                      offsets, pass_status, tickets, stream, nullptr, nullptr,
                      nullptr, gate);
@@ -532,6 +544,24 @@ inline hipError_t sort_pairs_cleared(const K *keys_in, u32 n, K *keys_a,
     }
   }
   return hipGetLastError();
+}
+
+// sort_pairs below, without its clearing launch and behind a gate.
+template <class K>
+inline hipError_t sort_pairs_cleared(const K *keys_in, u32 n, K *keys_a,
+                                     u32 *vals_a, K *keys_b, u32 *vals_b,
+                                     u32 *control, hipStream_t stream,
+                                     int block, const Gate &gate,
+                                     const u32 *vals_in = nullptr) {
+  constexpr int kPasses = passes_for<K>();
+  const Control c = control_layout(control, kPasses);
+  u32 *constant = gate.value || kPasses > 4 ? c.tickets + 32 : nullptr;
+  histogram_kernel<K, kPasses><<<hist_blocks_for(n), kThreads, 0, stream>>>(
+      keys_in, n, 0, c.rows, gate);
+  scan_kernel<<<kPasses, kRadix, 0, stream>>>(c.rows, kPasses, c.offsets, gate,
+                                              constant, n);
+  return sort_passes<K>(keys_in, n, keys_a, vals_a, keys_b, vals_b, control,
+                        stream, block, gate, constant, vals_in);
 }
 
 // Sorts n (key, position) pairs stably.  keys_in is read only; the sorted

@@ -511,6 +511,162 @@ __device__ __forceinline__ bool seg_dedupe(SegShared &sh,
   return true;
 }
 
+// ------------------------------------------------- builds of repeated keys
+// A build whose segments do not fit the LDS whole sorts by radix passes, unless
+// its segments fit once each has kept one update per key.  A sample of the keys
+// tells: S keys of D equally frequent ones hold about S^2 / 2D keys again, which
+// gives D, and the sample's digits give the largest segment's share of the
+// distinct keys (less what chance adds to the largest of 256 counts) and of all
+// updates.  It must not have more distinct keys than the table, nor many times
+// its share of the updates, which one workgroup reads.
+//
+// The sample is taken and judged by workgroups of the sort's own counting
+// launches, beside their others (a launch of one workgroup for all of it took 40
+// us).  Keys
+// are sampled in groups of four neighbours at places that follow no pattern; a
+// key that repeats inside its group (runs of equal keys) counts once.
+constexpr u32 kSampleKeys = 16384;
+constexpr u32 kSampleSlots = 1u << 17;
+constexpr u32 kSampleBlocks = kSampleKeys / rs::kThreads;
+
+// Device words of a sample: the table of its keys (0 = free; cleared before),
+// the keys, and what each was.
+struct BuildSample {
+  u32 table[kSampleSlots];
+  u32 keys[kSampleKeys];
+  u8 mark[kSampleKeys];  // kMarkUsed, kMarkNew
+};
+constexpr u64 kSampleClear = kSampleSlots;  // words to clear
+constexpr u64 kSampleWords = sizeof(BuildSample) / sizeof(u32);
+constexpr u32 kMarkUsed = 1, kMarkNew = 2;
+
+// The digit counts of a sort of 32-bit keys, and in the first kSampleBlocks
+// workgroups the sample.
+static __global__ __launch_bounds__(rs::kThreads) void build_count_kernel(
+    const u32 *__restrict__ keys, u32 n, u32 *__restrict__ rows,
+    BuildSample *sample) {
+  if (blockIdx.x >= kSampleBlocks) {
+    rs::histogram_block<u32, 4>(keys, n, 0, rows, blockIdx.x - kSampleBlocks,
+                                gridDim.x - kSampleBlocks);
+    return;
+  }
+  const u32 i = blockIdx.x * rs::kThreads + threadIdx.x;
+  u32 x = i / 4 * 0x9E3779B1u;
+  x = (x ^ (x >> 15)) * 0x85EBCA77u;
+  x = (x ^ (x >> 13)) * 0xC2B2AE3Du;
+  x ^= x >> 16;
+  const u32 key = keys[((u64(x) * (n / 4)) >> 32) * 4 + i % 4];
+  bool again = false;  // a lower lane of the group has the key
+#pragma unroll
+  for (u32 k = 1; k < 4; ++k) {
+    const u32 other = __shfl_xor(key, k, kWave);
+    again = again || (((i ^ k) & 3) < (i & 3) && other == key);
+  }
+  const bool used = !again && key;  // (0 marks the free slots)
+  // hot keys: one lane of a wave enters them
+  bool enter = used;
+  u64 open = ballot(used);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const u32 lead = open ? ffs64(open) - 1 : 0;
+    const bool same =
+        open && key == __shfl(key, static_cast<int>(lead), kWave);
+    if (same && lane_id() != lead) enter = false;
+    open &= ~ballot(same);
+  }
+  u32 mark = used ? kMarkUsed : 0;
+  if (enter) {
+    static_assert(kSampleSlots == 1u << 17, "hashes of 17 bits");
+    u32 h = (key * 0x9E3779B1u) >> 15;
+    while (true) {
+      const u32 cur = atomicCAS(&sample->table[h], 0u, key);
+      if (cur == 0) mark |= kMarkNew;
+      if (cur == 0 || cur == key) break;
+      h = (h + 1) & (kSampleSlots - 1);
+    }
+  }
+  sample->keys[i] = key;
+  sample->mark[i] = static_cast<u8>(mark);
+}
+
+// The digit offsets of the sort's four passes, and in the last workgroup the
+// decision: *choice and *choice_host (host memory) = 1 for segments, else 0.
+static __global__ __launch_bounds__(rs::kRadix) void build_scan_kernel(
+    const u32 *__restrict__ rows, u32 *__restrict__ offsets,
+    const BuildSample *__restrict__ sample, u32 *choice, u32 *choice_host) {
+  if (blockIdx.x < 4) {
+    rs::scan_block(rows, 4, blockIdx.x, offsets, nullptr, 0);
+    return;
+  }
+  constexpr u32 kEach = kSampleKeys / rs::kRadix / 4;
+  __shared__ u32 s_all[256], s_distinct[256];  // by digit, a key of each group
+  __shared__ u32 s_span, s_most[2], s_sum[2];
+  const u32 tid = threadIdx.x;
+  s_all[tid] = s_distinct[tid] = 0;
+  if (tid < 2) s_most[tid] = s_sum[tid] = 0;
+  if (tid == 0) s_span = 0;
+  uint4 key[kEach];
+  u32 mark[kEach];  // four to a word
+#pragma unroll
+  for (u32 j = 0; j < kEach; ++j) {
+    key[j] = reinterpret_cast<const uint4 *>(sample->keys)[j * rs::kRadix + tid];
+    mark[j] = reinterpret_cast<const u32 *>(sample->mark)[j * rs::kRadix + tid];
+  }
+  const u32 first = sample->keys[0];
+  u32 span = 0, used = 0, fresh = 0;
+#pragma unroll
+  for (u32 j = 0; j < kEach; ++j) {
+    span |= (key[j].x ^ first) | (key[j].y ^ first) | (key[j].z ^ first) |
+            (key[j].w ^ first);
+    used += __builtin_popcount(mark[j] & 0x01010101u * kMarkUsed);
+    fresh += __builtin_popcount(mark[j] & 0x01010101u * kMarkNew);
+  }
+#pragma unroll
+  for (int o = kWave / 2; o > 0; o >>= 1) span |= __shfl_xor(span, o, kWave);
+  used = wave_sum_u32(used);
+  fresh = wave_sum_u32(fresh);
+  __syncthreads();
+  if (lane_id() == 0) {
+    atomicOr(&s_span, span);
+    atomicAdd(&s_sum[0], used);
+    atomicAdd(&s_sum[1], fresh);
+  }
+  __syncthreads();
+  const u32 top = top_bit(s_span);
+  const u32 shift = top < 7 ? 0 : top - 7;
+#pragma unroll
+  for (u32 j = 0; j < kEach; ++j) {
+    const u32 d = (key[j].x >> shift) & 0xffu;
+    atomicAdd(&s_all[d], 1u);
+    if (mark[j] & kMarkNew) atomicAdd(&s_distinct[d], 1u);
+  }
+  __syncthreads();
+  u32 all = s_all[tid], distinct = s_distinct[tid];
+  atomicMax(&s_most[0], all);
+  atomicMax(&s_most[1], distinct);
+  distinct = wave_sum_u32(distinct);
+  __syncthreads();
+  if (tid == 0) s_span = 0;  // (its readers have passed a barrier)
+  __syncthreads();
+  if (lane_id() == 0) atomicAdd(&s_span, distinct);
+  __syncthreads();
+  if (tid) return;
+  const float taken = static_cast<float>(s_sum[0]);
+  const float again = taken - static_cast<float>(s_sum[1]);
+  const float total = 0.5f * taken * taken / (again > 1.0f ? again : 1.0f);
+  const float most = static_cast<float>(s_most[1]);
+  const float largest = total * (most - 2.5f * sqrtf(most)) /
+                        (static_cast<float>(s_span) + 1.0f);
+  // (0.85: the estimate is off by some 15% either way)
+  const u32 yes = s_most[0] <= kSampleKeys / 4 / 20 &&
+                          largest <= 0.85f * static_cast<float>(kHashMax)
+                      ? 1u
+                      : 0u;
+  *choice = yes;
+  __hip_atomic_store(choice_host, yes, __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // One workgroup per segment (ticket order = key order).  keys_in: the
 // batch (only its first key is read, for the shared high bits); pk/pp: the
 // partitioned keys and SegPayload payloads; tk/tp: scratch of n entries
