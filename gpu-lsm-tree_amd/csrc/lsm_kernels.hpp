@@ -1374,9 +1374,10 @@ __host__ __device__ __forceinline__ u32 range_queries_per_wave(u32 runs) {
 // allow while that keeps fewer than kRangeSpread waves busy (a few thousand
 // queries of a handful of runs would otherwise fill a fraction of the chip;
 // with more waves, narrow queries, whose waves then resolve a few bounds each
-// on mostly idle lanes, take a second turn on it).  12,000 ranges of 2^4 to
-// 2^24 keys over 6 million rows would gain from 8192 waves (2.3 -> 1.5 ms), but
-// 8,153 narrow ones over 240,860 rows then take 20 us instead of 11.
+// on mostly idle lanes, take a second turn on it).  12,000 sums of
+// 2^4 to 2^24 keys' width over 7.5 million rows in 4 runs would gain from 8192
+// waves (362 -> 244 us), but 8,153 of three rows over 240,860 rows in 3 runs then
+// take 16.7 us instead of 11.6.
 constexpr u64 kRangeSpread = 2048;
 inline u32 range_round(u64 n, u32 runs) {
   const u64 most = range_queries_per_wave(runs);
@@ -1397,13 +1398,19 @@ constexpr u32 kRangeOldStep = 1024;
 constexpr u32 kResolveRows = 512;
 constexpr u32 kResolveBlockRows = kRangeWaves * kResolveRows;
 
-// Runs from which on that is the faster way: a row of a newer run searches the
-// older ones one after another, two round trips each.  Sums of n ranges of w
-// rows, searching and resolving: 10 equal runs, n = 1, w = 60 23.3 and 16.9 us,
-// n = 10,000, w = 600 656 and 88; 40 runs 45 and 22, 9333 and 151; 4 runs 17.3
-// and 16.5, 266 and 106 (but n = 1, w = 3 14.7 and 15.4); 3 runs of falling size
-// n = 1025, w = 2000 47.9 and 63.0.
-constexpr u32 kResolveRuns = 4;
+// Whether that is the faster way for n ranges over so many runs: a row of a newer
+// run searches the older ones one after another, two round trips each.  Sums of n
+// ranges of w rows, searching and resolving: 10 equal runs, n = 1, w = 60 23.3 and
+// 16.9 us, n = 10,000, w = 600 656 and 88; 40 runs 45 and 22, 9333 and 151.  4 runs
+// are the edge, where few ranges are bound by the chain of one wave (falling
+// sizes, n = 1025, w = 200 21.5 and 22.8) and many by the searches (n = 10,000, w =
+// 600 270 and 112); over 3, n = 10,000, w = 2000 takes 247 and 271.
+constexpr u32 kResolveRuns = 5;
+constexpr u32 kResolveRunsMany = 4;
+constexpr u64 kResolveMany = 2048;
+__host__ __device__ __forceinline__ bool range_resolves(u64 n, u32 runs) {
+  return runs >= (n < kResolveMany ? kResolveRuns : kResolveRunsMany);
+}
 
 // Workgroups that share the long queries of one group of queries: `size` of
 // them, this one being number `rank`.  Where size > 1, acc and left (one each
@@ -1777,25 +1784,26 @@ __device__ __forceinline__ void range_resolve(typename T::K *keys, u32 *slots,
 // of a query's oldest run from its bounds when that run has no tombstones.
 // Sums are modulo 2^64 and are truncated to the value width.
 //
-// Over kResolveRuns runs or more (kResolve: compiled for them), queries with rows
-// of several runs search nothing up to kResolveBlockRows rows: a wave resolves
-// its short ones in LDS, as many at a time as fit, and the workgroup's waves one
-// of more than kResolveRows rows together (range_resolve).
+// With `resolve` (range_resolves; kResolve: compiled for it), queries with rows of
+// several runs search nothing up to kResolveBlockRows rows: a wave resolves its
+// short ones in LDS, as many at a time as fit, and the workgroup's waves one of
+// more than kResolveRows rows together (range_resolve).
 //
 // Bound by the searches, one per newer row and older run (directory entries,
 // then rows), whose lines come from beyond the L2 in a dictionary of tens of
-// megabytes, and by the rows read once.  12,000 sums (or counts) of 2^4 to
-// 2^24 keys' width over 6 million rows in 4 runs, a tenth tombstones: 0.54 ms
-// (9.4 ms when a wave answered each query and every row looked for newer
-// versions, in LDS or, beyond 2048 of them, in global memory); 16,384 counts
-// over one run of 2^20 rows 10 us (15).  A queue of all long queries' chunks
-// for a second launch took 0.38 ms, but its launch made every small call on a
-// large dictionary 3 to 5 us longer.
+// megabytes, and by the rows read once.  A launch of 12,000 sums (or counts) of
+// 2^4 to 2^24 keys' width over 6 million rows in 4 runs, a tenth tombstones: 0.72
+// ms (9 ms when a wave answered each query and every row looked for newer
+// versions, in LDS or, beyond 2048 of them, in global memory); 16,384 of up to 100
+// rows over one run of 2^20: counts 6.5 us (9.8), sums 12 (36).  A queue of all
+// long queries' chunks for a second launch made the wide ones some 30% faster,
+// but every small call on a large dictionary 3 to 5 us longer.
 template <class T, bool kResolve, class IO>
 __device__ __forceinline__ void range_block(const IO &io, u64 q_begin,
                                             u64 q_end, const RunSet<T> &runs,
                                             u64 group, u64 groups, u32 qw,
-                                            const RangeTeam &team) {
+                                            const RangeTeam &team,
+                                            bool resolve) {
   using K = typename T::K;
   constexpr u32 kSlots =
       2 * kMaxRuns > kWave ? 2 * kMaxRuns : static_cast<u32>(kWave);
@@ -1822,7 +1830,7 @@ __device__ __forceinline__ void range_block(const IO &io, u64 q_begin,
   __shared__ u32 s_list[kRangeWaves * kQMax];
   __shared__ u32 s_long[3];
   const u32 nr = runs.count;
-  const bool resolve = kResolve && nr >= kResolveRuns;
+  resolve = kResolve && resolve;
   __syncthreads();  // a previous call's readers of R are done
   R.load(runs);
   if (threadIdx.x < 3) s_long[threadIdx.x] = 0;
@@ -2104,7 +2112,7 @@ __global__ __launch_bounds__(kRangeThreads) void range_kernel(
   const IO io = io_arg.stage(s_io);  // range_block's first barrier orders it
   team.rank = blockIdx.x % team.size;
   range_block<T, kResolve>(io, 0, n, runs, blockIdx.x / team.size,
-                           gridDim.x / team.size, qw, team);
+                           gridDim.x / team.size, qw, team, kResolve);
 }
 
 // Smallest live key >= query, all-ones when there is none.

@@ -368,7 +368,7 @@ class LsmT : public HandleBase {
     const u64 waves = (n + qw - 1) / qw;
     const u32 groups = grid_for(waves, kRangeWaves, 1u << 16);
     const RangeTeam team = range_team(n, groups, rows, s);
-    if (set.count >= kResolveRuns)
+    if (range_resolves(n, set.count))
       range_kernel<T, true><<<groups * team.size, kRangeThreads, 0, s>>>(
           io, n, set, qw, team);
     else

@@ -333,7 +333,8 @@ __global__ __launch_bounds__(lsm::kRangeThreads) void step_query_kernel(
       lsm::range_block<T, true>(
           rio, r0, std::min<u64>(n_rng, r0 + kStepRangeChunk), runs, 0, 1,
           lsm::range_queries_per_wave(runs.count),
-          lsm::RangeTeam{1, 0, nullptr, nullptr});
+          lsm::RangeTeam{1, 0, nullptr, nullptr},
+          lsm::range_resolves(n_rng, runs.count));
     }
   }
 }
