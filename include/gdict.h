@@ -191,8 +191,9 @@ typedef struct gd_lsm_tuning {
                                       pair merges, 2..47 (10)              */
   uint32_t segmented_admission;    /* batches above small_batch_max: 1 =
                                       partition + per-segment LDS sort, radix
-                                      passes for larger builds (1), 2 = radix
-                                      passes + finalize; 0 = keep          */
+                                      passes for larger builds whose keys do
+                                      not repeat much (1), 2 = radix passes +
+                                      finalize; 0 = keep                   */
   uint32_t merge_block;            /* merge workgroup: 256 or 512 threads
                                       per tile (512)                       */
   uint32_t merge_ways;             /* most runs one merge pass takes: 2 =
