@@ -516,8 +516,8 @@ __device__ __forceinline__ bool seg_dedupe(SegShared &sh,
 // its segments fit once each has kept one update per key.  A sample of the keys
 // tells: S keys of D equally frequent ones hold about S^2 / 2D keys again, which
 // gives D, and the sample's digits give the largest segment's share of the
-// distinct keys (less what chance adds to the largest of 256 counts) and of all
-// updates.  It must not have more distinct keys than the table, nor many times
+// distinct keys (less what chance adds to the largest of 256 counts, but not below
+// an even share) and of all updates.  It must not have more distinct keys than the table, nor many times
 // its share of the updates, which one workgroup reads.
 //
 // The sample is taken and judged by workgroups of the sort's own counting
@@ -654,10 +654,13 @@ static __global__ __launch_bounds__(rs::kRadix) void build_scan_kernel(
   const float taken = static_cast<float>(s_sum[0]);
   const float again = taken - static_cast<float>(s_sum[1]);
   const float total = 0.5f * taken * taken / (again > 1.0f ? again : 1.0f);
+  const float distinct_sampled = static_cast<float>(s_span);
   const float most = static_cast<float>(s_most[1]);
-  const float largest = total * (most - 2.5f * sqrtf(most)) /
-                        (static_cast<float>(s_span) + 1.0f);
-  // (0.85: the estimate is off by some 15% either way)
+  const float even = distinct_sampled / 256.0f;
+  const float corrected = most - 2.5f * sqrtf(most);
+  const float largest = total * (corrected > even ? corrected : even) /
+                        (distinct_sampled + 1.0f);
+  // (0.85: the estimate is off by some 12% either way)
   const u32 yes = s_most[0] <= kSampleKeys / 4 / 20 &&
                           largest <= 0.85f * static_cast<float>(kHashMax)
                       ? 1u
